@@ -365,7 +365,7 @@ class HipContext:
 
     def set_dct_route(self, name):
         """Whole-matrix transform route: "auto" (the FFT route when both sides
-        allow it and the larger is at least 1024), "dense" or "fft"."""
+        allow it), "dense" or "fft"."""
         self.set_option(OPT_DCT_ROUTE, DCT_ROUTES[name])
 
     def set_pipeline_route(self, name):

@@ -179,6 +179,7 @@ void hh_context_destroy(hh_context *ctx) {
     if (ctx->d_scratch) (void)hipFree(ctx->d_scratch);
     hh::release_dct_resources(ctx);
     hh::release_fft_resources(ctx);
+    hh::release_line_tables(ctx);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

@@ -194,14 +194,34 @@ bool eo_candidate(const std::vector<Layer> &layers, uint32_t rows, uint32_t cols
            (a & (dtype == HH_F32 ? 15u : 7u)) == 0;
 }
 
-// hct3_decode_eo over the layers of a container whose bytes are at h_base
-// on the host and d_base on the device.
-int32_t decode_eo(hh_context *ctx, const std::vector<Layer> &layers, const uint8_t *h_base, const uint8_t *d_base,
-                  uint32_t rows, uint32_t cols, int32_t dtype, void *d_out, uint8_t *d_stage, hipStream_t s) {
+// Whether hct3_decode_lines takes a decode of these layers.
+bool lines_candidate(const hh_context *ctx, const std::vector<Layer> &layers, uint32_t rows, uint32_t cols) {
+    return ctx->dct_route != HH_DCT_DENSE && !layers.empty() && layers.size() <= 16 &&
+           hh::lines_supported(ctx, rows, cols, true);
+}
+
+std::vector<hh::Hct3Frag> device_frags(const std::vector<Layer> &layers, const uint8_t *h_base,
+                                       const uint8_t *d_base) {
     std::vector<hh::Hct3Frag> fr;
     for (const Layer &L : layers)
         fr.push_back(hh::Hct3Frag{d_base + (L.bitmap - h_base),
                                   d_base + (reinterpret_cast<const uint8_t *>(L.coef) - h_base), L.ncoef});
+    return fr;
+}
+
+// hct3_decode_lines over the layers of a container whose bytes are at
+// h_base on the host and d_base on the device.
+int32_t decode_lines(hh_context *ctx, const std::vector<Layer> &layers, const uint8_t *h_base, const uint8_t *d_base,
+                     uint32_t rows, uint32_t cols, int32_t dtype, void *d_out, hipStream_t s) {
+    const std::vector<hh::Hct3Frag> fr = device_frags(layers, h_base, d_base);
+    return hh::hct3_decode_lines(ctx, fr.data(), (uint32_t)fr.size(), false, rows, cols, dtype, d_out, s);
+}
+
+// hct3_decode_eo over the layers of a container whose bytes are at h_base
+// on the host and d_base on the device.
+int32_t decode_eo(hh_context *ctx, const std::vector<Layer> &layers, const uint8_t *h_base, const uint8_t *d_base,
+                  uint32_t rows, uint32_t cols, int32_t dtype, void *d_out, uint8_t *d_stage, hipStream_t s) {
+    const std::vector<hh::Hct3Frag> fr = device_frags(layers, h_base, d_base);
     return hh::hct3_decode_eo(ctx, fr.data(), (uint32_t)fr.size(), rows, cols, dtype, d_out, d_stage, s);
 }
 
@@ -247,8 +267,19 @@ int32_t hh_hct3_decompress(hh_context *ctx, const uint8_t *data, size_t len, con
     hh::DeviceGuard guard(ctx->device);
     if (guard.status() != hipSuccess) return from_hip(guard.status());
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (eo_candidate(layers, rows, cols, out_dtype, d_out)) {
+    if (lines_candidate(ctx, layers, rows, cols)) {
         // the container copied whole to the device, then decoded in place
+        rc = ensure_scratch(ctx, align16(len));
+        if (rc != HH_OK) return rc;
+        uint8_t *d_data = reinterpret_cast<uint8_t *>(ctx->d_scratch);
+        hipError_t e = hipMemcpyAsync(d_data, data, len, hipMemcpyHostToDevice, s);
+        if (e != hipSuccess) return from_hip(e);
+        rc = decode_lines(ctx, layers, data, d_data, rows, cols, out_dtype, d_out, s);
+        if (rc != HH_OK) return rc;
+        return from_hip(hipStreamSynchronize(s));
+    }
+    if (eo_candidate(layers, rows, cols, out_dtype, d_out)) {
+        // the same on the even / odd split or the long-row FFT
         const size_t st = stage_bytes(total, 0, 0);
         rc = ensure_scratch(ctx, st + align16(len));
         if (rc != HH_OK) return rc;
@@ -290,6 +321,9 @@ int32_t hh_hct3_decompress_device(hh_context *ctx, const uint8_t *h_data, const 
     if (!d_out) return HH_ERR_INVALID_ARGUMENT;
     hh::DeviceGuard guard(ctx->device);
     if (guard.status() != hipSuccess) return from_hip(guard.status());
+    if (lines_candidate(ctx, layers, rows, cols))
+        return decode_lines(ctx, layers, h_data, d_data, rows, cols, out_dtype, d_out,
+                            reinterpret_cast<hipStream_t>(stream));
     if (eo_candidate(layers, rows, cols, out_dtype, d_out)) {
         rc = ensure_scratch(ctx, stage_bytes(total, 0, 0));
         if (rc != HH_OK) return rc;
@@ -390,14 +424,28 @@ int32_t hh_spectral_reconstruct(hh_context *ctx, const uint8_t *const *frags, co
     // reconstruct (compressive.rs:728-752): one scatter with fragment 0's bitmap
     hh::DeviceGuard guard(ctx->device);
     if (guard.status() != hipSuccess) return from_hip(guard.status());
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    std::vector<Layer> layers{Layer{f0 + 24, coef.data(), ntot}};
+    if (lines_candidate(ctx, layers, h, w)) {
+        const size_t words = align16((size_t)bm);
+        int32_t rc = ensure_scratch(ctx, words + align16(coef.size()));
+        if (rc != HH_OK) return rc;
+        uint8_t *d_bits = reinterpret_cast<uint8_t *>(ctx->d_scratch), *d_coef = d_bits + words;
+        hipError_t e = hipMemcpyAsync(d_bits, f0 + 24, (size_t)bm, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess && ntot) e = hipMemcpyAsync(d_coef, coef.data(), coef.size(), hipMemcpyHostToDevice, s);
+        if (e != hipSuccess) return from_hip(e);
+        const hh::Hct3Frag F{d_bits, d_coef, ntot};
+        rc = hh::hct3_decode_lines(ctx, &F, 1, f32c != 0, h, w, out_dtype, d_out, s);
+        if (rc != HH_OK) return rc;
+        if (status) status->written = n;
+        return from_hip(hipStreamSynchronize(s));
+    }
     const size_t mat = align16((size_t)n * sizeof(float));
     int32_t rc = ensure_scratch(ctx, 2 * mat + stage_bytes(n, ntot, f32c));
     if (rc != HH_OK) return rc;
     uint8_t *base = reinterpret_cast<uint8_t *>(ctx->d_scratch);
     float *d_dense = reinterpret_cast<float *>(base);
     float *d_tmp = reinterpret_cast<float *>(base + mat);
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    std::vector<Layer> layers{Layer{f0 + 24, coef.data(), ntot}};
     rc = scatter_layers(layers, n, f32c, d_dense, base + 2 * mat, s);
     if (rc == HH_OK) rc = inverse_to(ctx, d_dense, d_tmp, h, w, out_dtype, d_out, s, !f32c);
     if (rc != HH_OK) return rc;
@@ -476,6 +524,8 @@ int32_t hh_idct_2d(hh_context *ctx, const float *d_in, uint32_t rows, uint32_t c
     hh::DeviceGuard guard(ctx->device);
     if (guard.status() != hipSuccess) return from_hip(guard.status());
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (hh::use_lines(ctx, rows, cols))
+        return hh::dct2d_lines(ctx, true, d_in, rows, cols, out_dtype, d_out, s);
     if (hh::use_fft(ctx, rows, cols) &&
         (reinterpret_cast<uintptr_t>(d_out) & (out_dtype == HH_F32 ? 15u : 7u)) == 0) {
         float *a, *b;
@@ -503,6 +553,7 @@ int32_t hh_dct_2d(hh_context *ctx, const float *d_in, uint32_t rows, uint32_t co
     hh::DeviceGuard guard(ctx->device);
     if (guard.status() != hipSuccess) return from_hip(guard.status());
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (hh::use_lines(ctx, rows, cols)) return hh::dct2d_lines(ctx, false, d_in, rows, cols, HH_F32, d_out, s);
     if (hh::use_fft(ctx, rows, cols) && ((reinterpret_cast<uintptr_t>(d_out) | reinterpret_cast<uintptr_t>(d_in)) & 15u) == 0) {
         float *a, *b;
         int32_t rc = hh::fft_scratch(ctx, total, s, &a, &b);

@@ -1,4 +1,5 @@
-// Whole-matrix DCT-II / DCT-III (orthonormal) in O(n^2 log n): a 1-D
+// Whole-matrix DCT-II / DCT-III (orthonormal) in O(n^2 log n) for sides
+// longer than dct_lines.hip holds in LDS (above 16384, up to 39936): a 1-D
 // transform along every row, a transpose, the 1-D transform along every
 // row of the transposed matrix, and a transpose back (converted to the
 // output type on the way).
@@ -764,9 +765,7 @@ bool fft_supported(uint32_t n) {
 
 bool use_fft(const hh_context *ctx, uint32_t rows, uint32_t cols) {
     if (ctx->dct_route == HH_DCT_DENSE) return false;
-    if (!fft_supported(rows) || !fft_supported(cols)) return false;
-    if (ctx->dct_route == HH_DCT_FFT) return true;
-    return (rows > cols ? rows : cols) >= kFftAutoMin;
+    return fft_supported(rows) && fft_supported(cols);
 }
 
 int32_t fft_scratch(hh_context *ctx, uint64_t total, hipStream_t s, float **a, float **b) {

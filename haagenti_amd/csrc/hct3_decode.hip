@@ -642,6 +642,13 @@ int32_t dct2d_full(hh_context *ctx, bool inverse, const float *d_in, float *d_tm
     if (rows == 0 || cols == 0) return HH_OK;
     const uint32_t h = rows, w = cols;
     const uint64_t total = (uint64_t)h * w;
+    if (use_lines(ctx, h, w)) {
+        const bool cvt = inverse && cvt_out != nullptr;
+        const int32_t rc = dct2d_lines(ctx, inverse, d_in, h, w, cvt ? cvt_dtype : HH_F32,
+                                       cvt ? cvt_out : static_cast<void *>(d_out), s);
+        if (rc == HH_OK && converted) *converted = cvt;
+        return rc;
+    }
     if (use_fft(ctx, h, w)) {
         const bool cvt = inverse && cvt_out != nullptr;
         void *out = cvt ? cvt_out : static_cast<void *>(d_out);

@@ -53,6 +53,7 @@ struct hh_context {
         uint64_t stamp = 0;
     };
     FftTables fft_tab[2];
+    FftTables line_tab[8];  // dct_lines.hip
     void *d_fft = nullptr;
     size_t fft_bytes = 0;
 };
@@ -297,16 +298,16 @@ int32_t dct2d_full(hh_context *ctx, bool inverse, const float *d_in, float *d_tm
                    int32_t cvt_dtype = HH_F32, void *cvt_out = nullptr, bool *converted = nullptr);
 void release_dct_resources(hh_context *ctx);
 
-// FFT route of the whole-matrix transforms (dct_fft.hip).  fft_supported:
-// n a multiple of 64 whose half factors into 2, 3, 5, 7 and fits in LDS.
-// use_fft: the route the context's setting takes for a rows x cols matrix
-// (HH_DCT_AUTO: both sides supported and the larger at least kFftAutoMin).
+// FFT route of the whole-matrix transforms for sides that dct_lines.hip does
+// not take, above 16384 (dct_fft.hip).  fft_supported: n a multiple of 64
+// whose half factors into 2, 3, 5, 7 and fits in LDS.  use_fft: whether a
+// rows x cols matrix takes it (both sides supported, the context's setting
+// not the dense products).
 // fft_scratch: two f32 matrices of `total` elements from the context.
 // dct2d_fft: the orthonormal 2-D DCT-II (forward) or DCT-III of the h x w
 // d_in into d_out (out_dtype; 16-byte aligned f32 or 8-byte aligned 16-bit;
 // the forward's d_in 16-byte aligned), with d_a and d_b (fft_scratch) as the
 // intermediates; d_in may be d_a.
-constexpr uint32_t kFftAutoMin = 1024;
 bool fft_supported(uint32_t n);
 bool use_fft(const hh_context *ctx, uint32_t rows, uint32_t cols);
 int32_t fft_scratch(hh_context *ctx, uint64_t total, hipStream_t s, float **a, float **b);
@@ -320,6 +321,23 @@ void release_fft_resources(hh_context *ctx);
 // a row's inputs past 8 per thread or past the LDS).
 int32_t hct3_decode_fft(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrags, uint32_t h, uint32_t w,
                         int32_t dtype, void *d_out, hipStream_t s);
+// The two-pass route (dct_lines.hip): rows, then columns, several lines per
+// workgroup.  lines_supported: both sides at most 16384 with no prime factor
+// above 127 (`frags`: and a row's bitmap words beside its points in LDS).
+// dct2d_lines: as dct2d_fft, its scratch the context's; no alignment is asked
+// beyond the element's.  hct3_decode_lines: the h x w HCT3 decode, the
+// fragments (values f16, or f32 with coef_f32) read by the row pass;
+// HH_ERR_UNSUPPORTED (nothing launched) outside those limits and for other
+// than 1..16 fragments.
+bool lines_supported(const hh_context *ctx, uint32_t h, uint32_t w, bool frags);
+inline bool use_lines(const hh_context *ctx, uint32_t h, uint32_t w) {
+    return ctx->dct_route != HH_DCT_DENSE && lines_supported(ctx, h, w, false);
+}
+int32_t dct2d_lines(hh_context *ctx, bool inverse, const float *d_in, uint32_t h, uint32_t w, int32_t out_dtype,
+                    void *d_out, hipStream_t s);
+int32_t hct3_decode_lines(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrags, bool coef_f32, uint32_t h,
+                          uint32_t w, int32_t dtype, void *d_out, hipStream_t s);
+void release_line_tables(hh_context *ctx);
 // zstd::decode_all on the host (host_zstd.cpp): false on a malformed stream.
 bool zstd_decode_all(const uint8_t *in, size_t len, std::vector<uint8_t> &out);
 

@@ -114,8 +114,8 @@ int32_t hh_context_synchronize(hh_context *ctx);
  * so a test can drive the path taken when a wait runs out.
  * HH_OPT_DCT_ROUTE picks the whole-matrix transform of hh_idct_2d,
  * hh_dct_2d and the HCT3 decode entries (hh_dct_route): HH_DCT_AUTO (the
- * default) takes the FFT route when both sides allow it and the larger is
- * at least 1024, the dense MFMA products otherwise.
+ * default) takes the FFT route when both sides allow it, the dense MFMA
+ * products otherwise.
  * HH_OPT_PIPELINE_ROUTE picks how hh_pipeline_submit decodes a unit's
  * tensors (hh_pipeline_route): HH_PIPE_AUTO (the default) decodes each
  * tensor with k >= 1024 whose blocks hold whole tiles in the fused launch
@@ -628,13 +628,13 @@ int32_t hh_turbo_tensor_decode(hh_context *ctx, const uint8_t *data, size_t len,
  * (crates/haagenti-cuda/src/dct_gpu.rs:1163-1227, 1404-1412): orthonormal
  * 2-D DCT-III of the row-major f32 d_in into d_out (out_dtype).  Two routes
  * (HH_OPT_DCT_ROUTE), as the reference switches to idct_2d_fft above 4096
- * (dct_gpu.rs:1081,1714-1722): an FFT route -- each side a multiple of 64
- * whose half has no prime factor above 7 and is at most 20480; every row
- * transformed by Makhoul's construction over an f32 FFT in LDS, a
- * transpose, the same along the other side, a transpose back -- and two
- * split-f16 MFMA products against cached DCT bases for every other shape
- * (both ~1e-6 x RMS; the 16-bit outputs are the round-to-nearest-even of
- * the f32 result).  Asynchronous on the stream. */
+ * (dct_gpu.rs:1081,1714-1722): an FFT route, Makhoul's construction over an
+ * f32 FFT in LDS along the rows and then the columns -- each side at most
+ * 16384 with no prime factor above 127, or (with transposes between) a
+ * multiple of 64 whose half has no prime factor above 7 and is at most 19968
+ * -- and two split-f16 MFMA products against cached DCT bases for every
+ * other shape (~2e-7 and ~1e-6 x RMS; the 16-bit outputs are the
+ * round-to-nearest-even of the f32 result).  Asynchronous on the stream. */
 int32_t hh_idct_2d(hh_context *ctx, const float *d_in, uint32_t rows, uint32_t cols, int32_t out_dtype,
                    void *d_out, void *stream);
 

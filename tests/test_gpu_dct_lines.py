@@ -1,0 +1,70 @@
+"""The two-pass whole-matrix transforms (csrc/dct_lines.hip) at the lengths
+where they can go wrong: one line, odd numbers of lines and lengths, every
+radix and the direct sums of the other primes, padded and unpadded LDS
+layouts, the longest lines, outputs that are not aligned; and HCT3 fragments
+whose rows start inside a bitmap byte.
+
+Bound: a length-N f32 FFT has a relative 2-norm error of about
+0.6 eps sqrt(log2 N) per pass (eps = 2^-24 roundings of the sums, as much
+again from the rounded twiddles), at most 1.4e-7 for N <= 2^14; a direct sum
+over p <= 127 terms adds about eps sqrt(p) / 2 = 3.4e-7.  Two passes in
+quadrature: below 5.2e-7, tested at 1e-6."""
+import numpy as np
+import pytest
+
+import gpu_util as G
+import oracle_lib as O
+from test_gpu_hct3 import H, dec, rel_err, route
+from test_oracle_hct3 import container, random_fragment
+
+pytestmark = pytest.mark.gpu
+REL = 1e-6
+
+
+def basis64(n):
+    T = G.torch()
+    k = T.arange(n, device="cuda")[:, None]
+    i = T.arange(n, device="cuda")[None, :]
+    m = T.cos((k * (2 * i + 1) % (4 * n)).double() * (np.pi / (2 * n))) * np.sqrt(2.0 / n)
+    m[0] = np.sqrt(1.0 / n)
+    return m
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 77), (2, 3), (16, 17), (37, 53), (127, 126), (143, 11), (48, 80),
+                                       (320, 448), (576, 576), (640, 1376), (2752, 96), (255, 1000), (16384, 34),
+                                       (33, 16384), (11008, 64), (64, 14336), (4096, 66)])
+def test_transforms_vs_f64(rows, cols):
+    T, h, c = G.torch(), H(), G.ctx()
+    x = T.randn(rows, cols, device="cuda", generator=T.Generator(device="cuda").manual_seed(rows + cols))
+    br, bc, xd = basis64(rows), basis64(cols), x.double()
+    fwd = T.empty(rows * cols, device="cuda")
+    inv = T.empty(rows * cols, device="cuda")
+    c.dct_2d(x, rows, cols, fwd, stream=G.stream())
+    c.idct_2d(x, rows, cols, inv, stream=G.stream())
+    for got, ref in ((fwd, br @ xd @ bc.t()), (inv, br.t() @ xd @ bc)):
+        e = float((got.view(rows, cols).double() - ref).norm() / ref.norm())
+        assert e <= REL, e
+    # 16-bit outputs are the rounding of the f32 result, at any element address
+    for dt, td in ((h.BF16, T.bfloat16), (h.F16, T.float16)):
+        for off in (0, 1):
+            out = T.full((rows * cols + 2,), 7.0, dtype=td, device="cuda")
+            c.idct_2d(x, rows, cols, out.data_ptr() + 2 * off, dtype=dt, stream=G.stream())
+            G.sync()
+            assert T.equal(out[off:off + rows * cols], inv.to(td))
+            assert bool((out[off + rows * cols:] == 7).all()) and (off == 0 or float(out[0]) == 7)
+
+
+@pytest.mark.parametrize("shape", [(97, 131), (64, 1000), (1000, 77), (1, 3000), (130, 2048)])
+def test_fragments_whose_rows_start_inside_a_byte(shape):
+    rng = np.random.default_rng(shape[0])
+    total = shape[0] * shape[1]
+    bm, v, _ = random_fragment(rng, total, 0.05)
+    data = container([random_fragment(rng, total, 0.3), (bm, v[:v.size // 2], None),
+                      random_fragment(rng, total, 0.01)])
+    rc, ref = O.hct3_decode(data, shape)
+    assert rc == O.OK
+    got = dec().decompress_to_gpu(data, shape).cpu().numpy()
+    assert rel_err(got, ref) <= 1e-5
+    with route("dense"):
+        dense = dec().decompress_to_gpu(data, shape).cpu().numpy()
+    assert rel_err(got, dense) <= 2e-5
