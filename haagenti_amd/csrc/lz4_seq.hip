@@ -10,8 +10,9 @@ __global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B) {
     using D = seq::SeqDec<R, S, false>;
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x;
-    const uint32_t b = blockIdx.x;
-    if (b >= B.nblocks) return;
+    if (blockIdx.x >= B.nblocks) return;
+    uint32_t b = blockIdx.x + B.first;
+    b = b >= B.nblocks ? b - B.nblocks : b;
 
     int32_t code = HH_OK, detail = HH_CORRUPT_NONE;
     uint64_t pos = 0, req = 0;
@@ -26,7 +27,8 @@ __global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B) {
     seq::lds8 *lds = (seq::lds8 *)smem;
     d.ring = lds;
     d.tab = reinterpret_cast<seq::lds32 *>(lds + R);
-    d.stage = lds + R + D::kTabLds + D::kSFront;
+    d.list = reinterpret_cast<seq::lds16 *>(lds + R + D::kTabLds);
+    d.stage = lds + R + D::kTabLds + D::kListLds + D::kSFront;
     d.gbuf = B.in;
     d.gsz = B.in_total;
     d.ioff = ioff;

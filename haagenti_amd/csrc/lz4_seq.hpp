@@ -6,6 +6,16 @@
 // them sharing a pass.  Used by the batched LZ4 kernel (lz4_seq.hip) and the
 // fused LZ4 -> tile kernel (hctt_decode.hip).
 //
+// What bounds it: one block is one wave's chain of dependent instructions
+// (7-10 cycles each when the wave is alone on its SIMD).  Tiles of 10 %
+// retention make ~1,400 sequences of ~10 bytes a 16 KiB block; a tensor of
+// 652 such blocks took 612 us when every sequence's header was read on its
+// own and matches were copied in runs up to the first that reads one of
+// them, 187 us with the tokens found by a walk (about 110 cycles a sequence),
+// one lane copying a sequence's literals and its match, and matches going as
+// soon as their own source bytes are there: 3.4 rounds a batch of 64.  At
+// 15 % 259 -> 123 us, at 20 % 95 -> 82 us.
+//
 // Semantics: crates/haagenti-lz4/src/block.rs:261-366 (decompress_block):
 // the same checks in the same order, the same reported positions, the early
 // stop once the output reaches output_size.  Every check is made by the
@@ -23,7 +33,8 @@
 //    16-byte loads; headers and literal runs are read there.  A batch ends
 //    where the stage does; a literal run or match that crosses a batch end
 //    continues in the next batch;
-//  * a 64-word table that maps a pass's chunks to their runs.
+//  * a table that maps a pass's chunks to their runs, or marks the output
+//    bytes of the matches still to be copied.
 // Copies write exactly their own bytes (16-byte chunks aligned in output
 // position; partial dwords merged with LDS and/or atomics), so the runs of a
 // pass may share chunks.  A match of length n at output position v with
@@ -49,6 +60,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // global read into one flat load, which is not ordered after earlier ds_*
 // writes of other lanes)
 typedef __attribute__((address_space(3))) uint8_t lds8;
+typedef __attribute__((address_space(3))) uint16_t lds16;
 typedef __attribute__((address_space(3))) uint32_t lds32;
 typedef __attribute__((address_space(3))) u32x4 ldsx4;
 
@@ -131,12 +143,21 @@ struct SeqDec {
     static constexpr uint32_t kSFront = 16;                // stage under-read (first chunk of a literal)
     static constexpr uint32_t kSPad = 32;                  // stage over-read (headers, realign)
     static constexpr uint32_t kStageLds = kSFront + S + kSPad;
-    static constexpr uint32_t kTabLds = 256;
-    // ring, table, stage (the caller may place them elsewhere)
-    static constexpr uint32_t kLds = R + kTabLds + kStageLds;
+    static constexpr uint32_t kTabWords = 112;
+    static constexpr uint32_t kTabLds = 4 * kTabWords;
+    static constexpr uint32_t kList = 256;
+    static constexpr uint32_t kListLds = 2 * kList;
+    // batches whose matches may run in any order (match_short): their output
+    // bytes each have a bit in the table, and one word after them
+    static constexpr uint32_t kShortBytes = 32 * (kTabWords - 1);
+    static constexpr uint32_t kShortLit = 32;    // longest literal run copied by one lane
+    static constexpr uint32_t kShortMatch = 18;  // longest match without a length extension
+    // ring, table, list, stage (the caller may place them elsewhere)
+    static constexpr uint32_t kLds = R + kTabLds + kListLds + kStageLds;
 
     lds8 *ring;
-    lds32 *tab;           // 64 words
+    lds32 *tab;           // kTabWords words
+    lds16 *list;          // kList token positions
     lds8 *stage;          // kSFront bytes of slack before it, kSPad after
     const uint8_t *gbuf;  // whole input buffer: every read is clamped to it
     uint64_t gsz;
@@ -451,6 +472,184 @@ struct SeqDec {
         }
     }
 
+    // ------------------------------------------------ short sequences
+    // Bytes from a token to the next when its match length has no extension
+    // and its literal length at most one byte (next: the byte after the
+    // token), else 0.
+    __device__ __forceinline__ static uint32_t short_dist(uint32_t token, uint32_t next) {
+        const uint32_t k = token >= 0xf0u ? 19u + next : (token >> 4) + 3u;
+        return (token & 15u) == 15u || (token >= 0xf0u && next == 255u) ? 0u : k;
+    }
+    // Finds the tokens of a run of such sequences from stage offset x0 on,
+    // each next token at or before stage offset xe and no window past x_max:
+    // their stage offsets go to the list, their number is returned, x0
+    // becomes the position after the last.
+    //
+    // The chain of headers is serial; what each link costs is kept small.
+    // 256 stage bytes at a time, register r of lane l holds where the next
+    // token is if one starts at byte 64 r + l (a multiple of 64 first), so a
+    // sequence is one readlane by the position itself and a bit set in a
+    // scalar mask; the positions then go to the list 64 at a time.
+    __device__ __forceinline__ uint32_t walk(uint32_t &x0, uint32_t xe, uint32_t x_max) const {
+        constexpr uint32_t kStop = 0xffffu;  // no short sequence here
+        uint32_t n = 0, x = x0;
+        bool on = true;
+        while (on && n + 96u <= kList && x <= x_max) {
+            const uint32_t wb = x & ~63u;
+            uint32_t nx[4];
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) {
+                const uint32_t p = wb + 64u * r + (uint32_t)lane;
+                const uint32_t a = p < xe ? p : 0u;
+                const uint32_t k = short_dist(stage[a], stage[a + 1u]);
+                nx[r] = k != 0u && p + k <= xe ? p + k : kStop;
+            }
+            uint64_t mask[4];
+            uint32_t o = x, last = x;
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) {
+                const uint32_t lim = wb + 64u * (r + 1u);
+                uint64_t m = 0;
+                while (o < lim) {
+                    last = o;
+                    m |= 1ull << (o & 63u);
+                    o = rdl(nx[r], o & 63u);
+                    if (o >= lim) break;
+                    last = o;
+                    m |= 1ull << (o & 63u);
+                    o = rdl(nx[r], o & 63u);
+                }
+                mask[r] = m;
+            }
+            if (o == kStop) {
+                const uint64_t keep = ~(1ull << (last & 63u));
+#pragma unroll
+                for (uint32_t r = 0; r < 4; r++)
+                    if ((last - wb) >> 6 == r) mask[r] &= keep;
+                o = last;
+                on = false;
+            }
+            x = o;
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) {
+                const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask[r] >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)mask[r], 0u));
+                if ((mask[r] >> lane) & 1ull) list[at] = (uint16_t)(wb + 64u * r + (uint32_t)lane);
+                n += (uint32_t)__builtin_popcountll(mask[r]);
+            }
+        }
+        wave_sync();
+        x0 = x;
+        return n;
+    }
+
+    // Each lane's literal run (n <= kShortLit bytes at stage offset src) to
+    // virtual position v, four bytes at a time.
+    __device__ __forceinline__ void lit_short(uint32_t v, uint32_t n, uint32_t src) const {
+        const lds32 *q = reinterpret_cast<const lds32 *>(stage + (src & ~3u));
+        const uint32_t sh = src & 3u;
+        uint32_t d0 = n > 0 ? q[0] : 0u;
+        for (uint32_t t = 0; ballot(t < n); t += 4) {
+            if (t < n) {
+                q++;
+                const uint32_t d1 = q[0];
+                const uint32_t w = __builtin_amdgcn_alignbyte(d1, d0, sh);
+                d0 = d1;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++)
+                    if (t + i < n) ring[(v + t + i) & kRM] = (uint8_t)(w >> (8 * i));
+            }
+        }
+    }
+
+    // The sources of the lanes' far matches (before rlo, in the written-out
+    // output), loaded as dwords: 9 bytes from any position.
+    struct FarSrc {
+        uint32_t d[3];
+    };
+    __device__ __forceinline__ uint32_t out_dword(int32_t w) const {
+        const int32_t lo = (int32_t)(a0 & ~3u), hi = (int32_t)((a0 + cap - 1u) & ~3u);
+        w = w < lo ? lo : w > hi ? hi : w;
+        return *reinterpret_cast<const uint32_t *>(obase + w);
+    }
+
+    // The batch's matches (lane: n <= kShortMatch bytes at virtual position v,
+    // offset off), in rounds: the output bytes of the matches not yet copied
+    // are marked in the table, and every match whose source bytes are clear of
+    // them copies, one lane each.  The first match left is always clear, so a
+    // round copies at least one; sources in the batch rarely chain more than a
+    // few deep.  vb: the batch's first virtual position.
+    __device__ __forceinline__ void match_short(uint32_t v, uint32_t n, uint32_t off, int32_t rlo, uint32_t vb,
+                                                const FarSrc &fs) const {
+        const bool live = n > 0;
+        const uint32_t r = live ? v - vb : 0u;
+        const uint64_t own = live ? ((1ull << n) - 1ull) << (r & 31u) : 0ull;
+        const uint32_t ow = r >> 5;
+        tab[lane] = 0u;
+        if (lane < (int)(kTabWords - 64u)) tab[64 + lane] = 0u;
+        wave_sync();
+        if (live) __hip_atomic_fetch_or(&tab[ow], (uint32_t)own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (own >> 32)
+            __hip_atomic_fetch_or(&tab[ow + 1], (uint32_t)(own >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        wave_sync();
+        // the source's part in this batch
+        const int32_t ss = (int32_t)(v - off), rs = ss - (int32_t)vb;
+        const int32_t re = rs + (int32_t)(off < n ? off : n);
+        const uint32_t cs = rs > 0 ? (uint32_t)rs : 0u;
+        const uint64_t need = live && re > 0 ? ((1ull << ((uint32_t)re - cs)) - 1ull) << (cs & 31u) : 0ull;
+        const uint32_t nw = need ? cs >> 5 : 0u;
+        const bool far = !LDS && ss < rlo, slow = n < 4u || n > 8u || off < n;
+        uint64_t pend = ballot(live);
+        while (pend) {
+            const uint64_t w = ((uint64_t)tab[nw + 1] << 32) | tab[nw];
+            const bool go = ((pend >> lane) & 1ull) && (w & need) == 0;
+            pend &= ~ballot(go);
+            if (go && !slow) {
+                // 4 to 8 bytes, not periodic: three dwords hold them
+                uint32_t d[3];
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+                    d[i] = *reinterpret_cast<const lds32 *>(ring + ((((uint32_t)ss & ~3u) + 4u * i) & kRM));
+                if (!LDS) {
+#pragma unroll
+                    for (int i = 0; i < 3; i++) d[i] = far ? fs.d[i] : d[i];
+                }
+                const uint32_t x = __builtin_amdgcn_alignbyte(d[1], d[0], (uint32_t)ss & 3u);
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) ring[(v + i) & kRM] = (uint8_t)(x >> (8 * i));
+                if (n > 4u) {
+                    const uint32_t y = __builtin_amdgcn_alignbyte(d[2], d[1], (uint32_t)ss & 3u);
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; i++)
+                        if (4u + i < n) ring[(v + 4u + i) & kRM] = (uint8_t)(y >> (8 * i));
+                }
+            }
+            if (go && slow) {
+                // byte t from source byte t mod off
+                uint32_t m = 0;
+                for (uint32_t t = 0; t < n; t++) {
+                    uint32_t b;
+                    if (far) {
+                        const uint32_t w = out_dword((ss + (int32_t)t) & ~3);
+                        b = w >> (8u * ((uint32_t)(ss + (int32_t)t) & 3u));
+                    } else {
+                        b = ring[((uint32_t)ss + m) & kRM];
+                    }
+                    ring[(v + t) & kRM] = (uint8_t)b;
+                    m = m + 1u == off ? 0u : m + 1u;
+                }
+            }
+            wave_sync();
+            if (pend && go) {
+                __hip_atomic_fetch_and(&tab[ow], ~(uint32_t)own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (own >> 32)
+                    __hip_atomic_fetch_and(&tab[ow + 1], ~(uint32_t)(own >> 32), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            wave_sync();
+        }
+    }
+
     // Copies one parsed batch: lane i < nsl holds slot i (a literal run of
     // ll bytes at stage offset ls, then a match of ml bytes at offset mo);
     // the batch starts at output position op_b and ends at op.
@@ -560,7 +759,26 @@ struct SeqDec {
             return;
         }
         // short runs: all literal runs of the batch at once, then the matches
-        run_pass<false>(vl, ll, ls, live, rlo);
+        const bool short_m = op - op_b <= kShortBytes && ballot(ml > kShortMatch) == 0;
+        FarSrc fs;
+        if (short_m && !LDS) {
+            // far sources are final: their loads run beside the literal copies
+            const int32_t ss = (int32_t)(vm - mo);
+            if (ml > 0 && ss < rlo) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) fs.d[i] = out_dword((ss & ~3) + 4 * i);
+            }
+        }
+        if (ballot(ll > kShortLit) == 0) {
+            lit_short(vl, ll, ls);
+            wave_sync();
+        } else {
+            run_pass<false>(vl, ll, ls, live, rlo);
+        }
+        if (short_m) {
+            match_short(vm, ml, mo, rlo, op_b + a0, fs);
+            return;
+        }
         // matches in order; a pass takes the next pending match and every
         // following one up to the first whose source reaches past the start
         // of that first match
@@ -627,13 +845,14 @@ struct SeqDec {
 // out the rest of a successful block (d.flush(true)).  `staged`: the caller
 // has already put the stage for input position 0 in place.
 //
-// A batch is parsed in two ways.  The fast loop only follows the chain of
-// headers -- token, literal length, offset, match length -- and records
-// each sequence in a lane, stopping where a header would leave the stage or
-// a length extension is longer than 7 (6) bytes; the wave then checks all of
-// the recorded sequences at once (input bounds, capacity, offsets, the
-// batch budget) and keeps those before the first one that fails.  The
-// general step parses the sequence after them one state at a time with
+// A batch is parsed in three ways.  Runs of short sequences come from a walk
+// over their tokens (SeqDec::walk), each lane then reading its sequence's
+// fields; between them the fast loop follows the chain of headers -- token,
+// literal length, offset, match length -- and records each sequence in a
+// lane, stopping where a header would leave the stage or a length extension
+// is longer than 7 (6) bytes.  The wave then checks all of the recorded
+// sequences at once (input bounds, capacity, offsets, the batch budget) and
+// keeps those before the first one that fails.  The general step parses the sequence after them one state at a time with
 // every check in the reference's order: a run continued from the previous
 // batch, a run cut by the stage end or the budget, long extensions, and
 // every error, reported as the reference reports it.
@@ -650,6 +869,8 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
     uint32_t lit_rem = 0, m_rem = 0, m_off = 0, tml = 0;
     d.hv = 0;
     d.hb = 0;
+    // the list of short sequences: next entry, entries, stage offset after them
+    uint32_t li = 0, ln = 0, lx = 0;
     d.pf_on = false;
     if (end == 0) return;
     if (!staged)
@@ -668,6 +889,8 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
         // slots in lanes (slot i in lane i): literal stage offset and length,
         // match offset and length, token position (fast loop only)
         uint32_t ls = 0, ll = 0, mo = 0, ml = 0, tp = 0;
+        uint64_t walked = 0;  // slots of sequences from the list
+        uint32_t lslot = 64, lfirst = 0;  // the list's first slot of this batch and its entry
         if (ms != kToken) nsl = 1;  // a run continued from the previous batch
         for (;;) {
             // ---- fast loop: header chain only
@@ -683,53 +906,106 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                 uint32_t fo = op;
                 uint32_t fl = lim < op_b + D::kOB ? lim : op_b + D::kOB;
                 bool full = false;
-                while (nsl < 64u && fp <= hl) {
-                    if (!d.in_win8(fp)) d.read16(fp);
-                    const uint64_t t8 = d.peek8(fp);
-                    const uint32_t token = (uint32_t)t8 & 0xffu;
-                    uint32_t lit = token >> 4;
-                    uint32_t p = fp + 1;
-                    if (lit == 15u) {
-                        const uint64_t x = t8 >> 8;
-                        const uint32_t e = (uint32_t)__builtin_ctzll(~x | (1ull << 56)) >> 3;  // 7: none
-                        if (e == 7u) break;
-                        lit += 255u * e + (uint32_t)((x >> (8 * e)) & 0xffu);
-                        p += e + 1;
+                // short sequences end inside the stage and the block
+                const uint32_t we = d.at_end || end - d.sb < S ? end - d.sb : S;
+                for (;;) {
+                    // short sequences, up to 64 at once from the list
+                    const uint32_t w0 = nsl;
+                    if (nsl < 64u && fp <= hl && fo < fl) {
+                        if (li == ln) {
+                            if (!d.in_win8(fp)) d.read16(fp);
+                            const uint32_t t2 = (uint32_t)d.peek8(fp) & 0xffffu;
+                            const uint32_t k = D::short_dist(t2 & 0xffu, t2 >> 8);
+                            if (k != 0u && fp - d.sb + k <= we) {
+                                // (their output is at least their input: no
+                                // token past the batch's budget)
+                                lx = fp - d.sb;
+                                ln = d.walk(lx, we, lx + (fl - fo));
+                                li = 0;
+                            }
+                        }
+                        if (li < ln) {
+                            const uint32_t n = ln - li < 64u - nsl ? ln - li : 64u - nsl;
+                            const bool me = lane >= w0 && lane < w0 + n;
+                            if (me) {
+                                tp = d.list[li + (lane - w0)];
+                                const uint32_t token = d.stage[tp], next = d.stage[tp + 1u];
+                                const bool x1 = token >= 0xf0u;
+                                ls = tp + (x1 ? 2u : 1u);
+                                ll = x1 ? 15u + next : token >> 4;
+                                ml = (token & 15u) + 4u;
+                                mo = (uint32_t)d.stage[ls + ll] | ((uint32_t)d.stage[ls + ll + 1u] << 8);
+                                tp += d.sb;
+                            }
+                            fo += rdl(scan_add(me ? ll + ml : 0u), 63);
+                            walked |= (~0ull >> (64u - n)) << w0;
+                            lslot = w0;
+                            lfirst = li;
+                            li += n;
+                            nsl += n;
+                            fp = d.sb + (li < ln ? rfl((uint32_t)d.list[li]) : lx);
+                        }
                     }
-                    const uint32_t le = p + lit;  // offset position
-                    if (le > hl) break;
-                    if (!d.in_win8(le)) d.read16(le);
-                    const uint64_t o8 = d.peek8(le);
-                    uint32_t mlen = (token & 15u) + 4u;
-                    uint32_t q = le + 2;
-                    if ((token & 15u) == 15u) {
-                        const uint64_t x = o8 >> 16;
-                        const uint32_t e = (uint32_t)__builtin_ctzll(~x | (1ull << 48)) >> 3;  // 6: none
-                        if (e == 6u) break;
-                        mlen += 255u * e + (uint32_t)((x >> (8 * e)) & 0xffu);
-                        q += e + 1;
+                    // then the others, one at a time, until a short one
+                    // follows
+                    bool back = false, any = false;
+                    while (nsl < 64u && fp <= hl) {
+                        if (!d.in_win8(fp)) d.read16(fp);
+                        const uint64_t t8 = d.peek8(fp);
+                        const uint32_t token = (uint32_t)t8 & 0xffu;
+                        uint32_t lit = token >> 4;
+                        if (any && fo < fl) {
+                            const uint32_t k = D::short_dist(token, (uint32_t)(t8 >> 8) & 0xffu);
+                            if (k != 0u && fp - d.sb + k <= we) {
+                                back = true;
+                                break;
+                            }
+                        }
+                        any = true;
+                        uint32_t p = fp + 1;
+                        if (lit == 15u) {
+                            const uint64_t x = t8 >> 8;
+                            const uint32_t e = (uint32_t)__builtin_ctzll(~x | (1ull << 56)) >> 3;  // 7: none
+                            if (e == 7u) break;
+                            lit += 255u * e + (uint32_t)((x >> (8 * e)) & 0xffu);
+                            p += e + 1;
+                        }
+                        const uint32_t le = p + lit;  // offset position
+                        if (le > hl) break;
+                        if (!d.in_win8(le)) d.read16(le);
+                        const uint64_t o8 = d.peek8(le);
+                        uint32_t mlen = (token & 15u) + 4u;
+                        uint32_t q = le + 2;
+                        if ((token & 15u) == 15u) {
+                            const uint64_t x = o8 >> 16;
+                            const uint32_t e = (uint32_t)__builtin_ctzll(~x | (1ull << 48)) >> 3;  // 6: none
+                            if (e == 6u) break;
+                            mlen += 255u * e + (uint32_t)((x >> (8 * e)) & 0xffu);
+                            q += e + 1;
+                        }
+                        const uint32_t off = (uint32_t)o8 & 0xffffu;
+                        const uint32_t fm = fo + lit;
+                        uint32_t fl2 = fl;
+                        if (!LDS && off <= R - 128u && off <= fm) {
+                            const uint32_t l2 = fm - off + (R - 64u);
+                            fl2 = l2 < fl2 ? l2 : fl2;
+                        }
+                        if (fm + mlen > fl2) {
+                            full = true;
+                            break;
+                        }
+                        const bool me = lane == nsl;
+                        tp = me ? fp : tp;
+                        ls = me ? p - d.sb : ls;
+                        ll = me ? lit : ll;
+                        mo = me ? off : mo;
+                        ml = me ? mlen : ml;
+                        nsl++;
+                        fp = q;
+                        fo = fm + mlen;
+                        fl = fl2;
                     }
-                    const uint32_t off = (uint32_t)o8 & 0xffffu;
-                    const uint32_t fm = fo + lit;
-                    uint32_t fl2 = fl;
-                    if (!LDS && off <= R - 128u && off <= fm) {
-                        const uint32_t l2 = fm - off + (R - 64u);
-                        fl2 = l2 < fl2 ? l2 : fl2;
-                    }
-                    if (fm + mlen > fl2) {
-                        full = true;
-                        break;
-                    }
-                    const bool me = lane == nsl;
-                    tp = me ? fp : tp;
-                    ls = me ? p - d.sb : ls;
-                    ll = me ? lit : ll;
-                    mo = me ? off : mo;
-                    ml = me ? mlen : ml;
-                    nsl++;
-                    fp = q;
-                    fo = fm + mlen;
-                    fl = fl2;
+                    if (!back) break;
                 }
                 if (nsl > f0) {
                     // check slots f0 .. nsl - 1 at once; keep those before
@@ -741,11 +1017,15 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                     const uint32_t qn = bperm(tp, lane + 1u);
                     const uint32_t q = lane + 1u == nsl ? fp : qn;  // input end of each slot
                     // near-match limit: prefix minimum over the fast slots
-                    uint32_t nl = (!LDS && lane >= f0 && live && mo <= R - 128u) ? om - mo + (R - 64u) : 0xffffffffu;
+                    // (a walked sequence's match does not end the batch for a
+                    // source that leaves the ring: it reads the output)
+                    uint32_t nl = (!LDS && lane >= f0 && live && mo <= R - 128u && !((walked >> lane) & 1ull))
+                                      ? om - mo + (R - 64u)
+                                      : 0xffffffffu;
                     nl = ~scan_max(~nl);
                     nl = nl < lim ? nl : lim;
-                    const bool ok = q <= end && om < cap && mo != 0u && mo <= om && oe <= cap && oe - op_b <= D::kOB &&
-                                    oe <= nl;
+                    const bool valid = q <= end && om < cap && mo != 0u && mo <= om && oe <= cap;
+                    const bool ok = valid && oe - op_b <= D::kOB && oe <= nl;
                     const uint64_t badm = ballot(!ok && lane >= f0 && live);
                     const uint32_t f = badm ? (uint32_t)__builtin_ctzll(badm) : nsl;
                     if (f > f0) {
@@ -753,8 +1033,16 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                         lim = rdl(nl, f - 1u);
                         bout = op - op_b;
                     }
-                    if (f < nsl) full = false;
+                    // a slot past the batch's budget or limit starts the next batch
+                    if (f < nsl) full = (ballot(valid) >> f) & 1ull;
                     ip = f < nsl ? rdl(tp, f) : fp;
+                    // the list goes on with the first slot not kept
+                    if (f < nsl && li > 0) {
+                        if (lslot <= f && lslot < nsl)
+                            li = lfirst + (f - lslot);
+                        else
+                            li = ln = 0;
+                    }
                     nsl = f;
                     const bool keep = lane < f;
                     ls = keep ? ls : 0u;
@@ -965,7 +1253,10 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
         // operations complete in order)
         d.op = op;
         if (bout > 0) d.execute(nsl, op_b, ls, ll, mo, ml);
-        if (restage) d.restage(ip);
+        if (restage) {
+            d.restage(ip);
+            li = ln = 0;
+        }
         if (bout > 0) {
             d.flush(false);
             progress(op);

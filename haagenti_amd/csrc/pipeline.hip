@@ -689,7 +689,8 @@ int32_t hh_pipeline_submit(hh_pipeline *p, const uint8_t *h_data, size_t len, co
         // the tile scratch: a short block's tail zeroed, as in the fused launch
         const hh::Lz4Batch B = {s.d_in, len, d_in_off + f, d_in_len + f, lz4_out,
                                 d_lz4_out ? lz4_cap : tiles_total, d_out_off + f, d_out_cap + f, nb2,
-                                s.d_status + f, d_lz4_out ? 0u : 1u};
+                                s.d_status + f, d_lz4_out ? 0u : 1u,
+                                hh::lz4_first_block(rest.data(), (uint32_t)rest.size(), nb2)};
         e = hh::launch_lz4_batch(B, hh::lz4_decoder_for_tiles(p->ctx, rest.data(), (uint32_t)rest.size()),
                                  p->compute);
         if (e != hipSuccess) return from_hip(e);

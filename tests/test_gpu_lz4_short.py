@@ -1,0 +1,98 @@
+"""Blocks of many short LZ4 sequences on the sequence-batched decoder
+(csrc/lz4_seq.hpp), against the oracle: the edges of what its token walk
+takes (literal lengths without, with one and with two extension bytes, match
+lengths without and with one), more sequences than its list and a batch
+hold, tokens on every position of the 64-byte windows and of the stage's
+end, matches that chain through one batch, repeat their own bytes or reach
+back past the ring; and tiles of very low retention through both layer
+routes."""
+import numpy as np
+import pytest
+
+import gpu_util as G
+import oracle_lib as O
+from test_gpu_lz4 import _seq, check_against_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True, params=["seq", "seq8"])
+def decoder(request):
+    G.ctx().set_lz4_decoder(request.param)
+    yield request.param
+    G.ctx().set_lz4_decoder("auto")
+
+
+def stream(rng, nseq, lits, mls, offs):
+    """nseq sequences with lengths and offsets drawn from the given lists
+    (an offset is kept within the output), ending with literals."""
+    out, size = bytearray(_seq(bytes(rng.integers(0, 256, 40, dtype=np.uint8)), 7, 5)), 45
+    for _ in range(nseq):
+        n, m = int(rng.choice(lits)), int(rng.choice(mls))
+        off = min(int(rng.choice(offs)), size + n)
+        out += _seq(bytes(rng.integers(0, 256, n, dtype=np.uint8)), off, m)
+        size += n + m
+    tail = bytes(rng.integers(0, 256, 9, dtype=np.uint8))
+    return bytes(out + _seq(tail)), size + 9
+
+
+CASES = {
+    "shortest": ([0], [4], [1, 2, 3, 4, 5, 60, 300]),
+    "no_extension": (range(0, 15), range(4, 19), range(1, 400)),
+    "one_literal_byte": ([0, 3, 14, 15, 16, 100, 268, 269], [4, 5, 18], range(1, 3000)),
+    "two_literal_bytes": ([5, 269, 270, 271, 524, 525], [4, 9], range(1, 3000)),
+    "match_extension": ([0, 1, 7], [4, 18, 19, 20, 270, 273, 274], [1, 2, 5, 17, 400]),
+    "chained": ([0, 1, 2], [4, 5, 8], [4, 5, 6, 7, 8]),
+    "far": ([2, 6, 9], [4, 5, 8, 9, 10, 18], [3900, 4000, 4032, 4064, 4096, 8100, 8192, 12000]),
+}
+
+
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_short_sequences(case):
+    lits, mls, offs = (list(x) for x in CASES[case])
+    rng = np.random.default_rng(sorted(CASES).index(case))
+    items = [stream(rng, n, lits, mls, offs) for n in (1, 3, 62, 63, 64, 65, 127, 200, 255, 256, 257, 1500)]
+    # every start within a window, and lengths that move the stage's ends
+    items += [stream(rng, 700 + i, lits, mls, offs) for i in range(24)]
+    streams, caps = [s for s, _ in items], [c for _, c in items]
+    for in_align, out_align in ((0, 0), (5, 11)):
+        check_against_oracle(streams, caps, in_align=in_align, out_align=out_align, in_pad=in_align, out_pad=3)
+    # a capacity that ends inside a batch, and damaged bytes: the same records
+    check_against_oracle(streams, [c * 2 // 3 for c in caps], out_pad=3)
+    broken = []
+    for s in streams:
+        b = bytearray(s)
+        b[int(rng.integers(len(b) // 3, len(b)))] ^= int(rng.integers(1, 256))
+        broken.append(bytes(b))
+    check_against_oracle(broken, caps, out_pad=3)
+
+
+@pytest.mark.parametrize("rho", [0.05, 0.10, 0.15, 0.20])
+def test_sparse_tiles_on_both_routes(rho):
+    import haagenti_amd as H
+    from layer_util import encode_layer
+    T = G.torch()
+    k = H.hctt_retain_count(rho)
+    shapes = [("a", 256, 1024), ("b", 640, 512)]
+    L = encode_layer(H, shapes, [k, H.hctt_retain_count(0.3)], 11, 16352)
+    d_in, n = G.dev(L["blob"]), L["in_off"].size
+    st = T.zeros(n * 32, dtype=T.uint8, device="cuda")
+    scratch = T.zeros(L["scratch_bytes"], dtype=T.uint8, device="cuda")
+    two = [T.empty(t["rows"] * t["cols"], dtype=T.float32, device="cuda") for t in L["tensors"]]
+    one = [T.empty_like(o) for o in two]
+    G.ctx().hctt_decode_lz4_batch(
+        d_in, d_in.numel(), G.dev(L["in_off"]), G.dev(L["in_len"]), scratch, G.dev(L["out_off"]), G.dev(L["out_cap"]),
+        n, st, [(scratch.data_ptr() + t["soff"], t["tiles"].size, t["rows"], t["cols"], t["k"], o)
+                for t, o in zip(L["tensors"], two)], stream=G.stream())
+    G.sync()
+    want = np.concatenate([t["tiles"].ravel() for t in L["tensors"]])
+    assert np.array_equal(G.host_u8(scratch), want)
+    rc = G.ctx().hctt_decode_lz4_fused(
+        d_in, d_in.numel(), G.dev(L["in_off"]), G.dev(L["in_len"]), n, st,
+        [(t["rows"], t["cols"], t["k"], o) for t, o in zip(L["tensors"], one)],
+        [16352 // H.hctt_tile_bytes(t["k"]) for t in L["tensors"]], stream=G.stream())
+    assert rc == H.OK
+    G.sync()
+    assert (G.host_u8(st).view(np.int32)[0::8] == 0).all()
+    for a, b in zip(two, one):
+        assert T.equal(a, b)
