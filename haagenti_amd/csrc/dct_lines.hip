@@ -15,19 +15,21 @@
 // in LDS as a Stockham autosort FFT in f32 (radix 16, 8, 4, 2, 3, 5, 7, then
 // other primes up to 127 as direct sums), twiddles rounded from double.
 //
-// The row pass writes its result in panels [h / G][w][G] of its G = 2 PC
-// rows: a workgroup's output is one contiguous run, and the column pass,
-// whose lines are 2 PC columns, reads 2 PC G neighbouring values at a time.
-// The column pass writes the row-major result, 2 PC elements of a row at a
-// time; workgroups of neighbouring columns are placed on one XCD so that
-// its L2 joins their writes into whole lines.
+// The row pass writes its result in panels [h / G][w][G] of G rows, its own
+// 2 PC or those of two or four workgroups of one XCD (panel_share): the
+// column pass, whose lines are 2 PC columns, reads 2 PC G neighbouring values
+// at a time.  The column pass writes the row-major result, 2 PC elements of
+// a row at a time; workgroups of neighbouring columns are placed on one XCD
+// so that its L2 joins their writes into whole lines.  Where a workgroup
+// holds two columns only (more than 8192 rows), it writes them as panels and
+// untangle_kernel makes rows of them through LDS tiles (through_panels).
 //
 // What bounds it: each pass reads and writes the matrix once (4096 x 4096 to
 // bf16: 64 + 64 + 64 + 32 MB, 36 us at the device copy's 6.3 TB/s); a pass
 // takes 42-43 us there, its workgroups' loads, ~1,100 VALU instructions per
 // wave and stores one after the other (VALU ~40 % busy).  Against the row
 // transforms and transposes of dct_fft.hip (four passes over f32 matrices):
-// 4096 x 4096 87 against 141 us, 14336 x 4096 forward 553 against 637 us; and
+// 4096 x 4096 87 against 141 us, 14336 x 4096 forward 432 against 638 us; and
 // against the dense products, which shapes below 1024 and sides with other
 // primes took: 576 x 576 18 against 105 us, 3000 x 1280 44 against 330 us --
 // so every shape this file supports takes it.
@@ -65,7 +67,8 @@ struct Lines {
     uint32_t gsh;     // log2 of the panels' height G (kSrcPanels)
     uint32_t pcs;     // log2 of the pairs of lines per workgroup
     uint32_t psh;     // LDS: point x at slot x + (x >> psh)
-    uint32_t per_xcd; // column pass: workgroups per XCD (0: not placed)
+    uint32_t per_xcd; // workgroups per XCD (0: not placed)
+    uint32_t msh;     // kDstPanels: log2 of the workgroups that fill a panel
     uint32_t nr;
     uint64_t radix[2]; // a byte each, in order (kept in scalar registers)
     // kSrcFrags: fragment f's bitmap (bit row N + n), values and per-row set
@@ -75,6 +78,12 @@ struct Lines {
     const uint8_t *coef[kMaxFrags];
     const uint32_t *counts[kMaxFrags];
     uint32_t ncoef[kMaxFrags];
+};
+
+struct Untangle {
+    const float *in;
+    void *out;
+    uint32_t N, lines, pcs;
 };
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
@@ -238,8 +247,9 @@ struct Dft<7, INV> {
 // 32-bit lane offset then takes no address arithmetic per lane (the empty
 // asm keeps the compiler from adding the lane offset first)
 typedef __attribute__((address_space(1))) uint8_t glb8;
+__device__ __forceinline__ glb8 *global(const void *p) { return (glb8 *)(uintptr_t)p; }
 __device__ __forceinline__ glb8 *scalar_ptr(const void *base, int64_t bytes) {
-    glb8 *b = (glb8 *)(uintptr_t)base + bytes;
+    glb8 *b = global(base) + bytes;
     __asm__("" : "+s"(b));
     return b;
 }
@@ -248,9 +258,39 @@ template <class V>
 __device__ __forceinline__ V ld_s(const void *base, int64_t bytes, uint32_t lane_bytes) {
     return *(__attribute__((address_space(1))) const V *)(scalar_ptr(base, bytes) + (size_t)lane_bytes);
 }
-template <class V>
-__device__ __forceinline__ void st_s(glb8 *b, uint32_t lane_bytes, V v) {
+template <class I, class V>
+__device__ __forceinline__ void st_s(glb8 *b, I lane_bytes, V v) {
     *(__attribute__((address_space(1))) V *)(b + (size_t)lane_bytes) = v;
+}
+// Neighbouring elements v of a row (kDstPanels: a pair) to o[at]: vec as one
+// store, else each in its own, the second one only if it is there.
+template <int DST, class I>
+__device__ __forceinline__ void store_pair(glb8 *o, I at, bool vec, bool second, float2 v) {
+    const I x = at * (DST == kDstPanels ? 8 : DST == HH_F32 ? 4 : 2);
+    if constexpr (DST == kDstPanels) {
+        st_s(o, x, f32x2{v.x, v.y});
+    } else if constexpr (DST == HH_F32) {
+        if (vec) {
+            st_s(o, x, f32x2{v.x, v.y});
+        } else {
+            st_s(o, x, v.x);
+            if (second) st_s(o, x + 4u, v.y);
+        }
+    } else {
+        uint32_t b;
+        if constexpr (DST == HH_BF16) {
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+            b = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v.x, (__bf16)v.y});
+        } else {
+            b = f32_to_f16_bits(v.x) | (f32_to_f16_bits(v.y) << 16);
+        }
+        if (vec) {
+            st_s(o, x, b);
+        } else {
+            st_s(o, x, (uint16_t)b);
+            if (second) st_s(o, x + 2u, (uint16_t)(b >> 16));
+        }
+    }
 }
 // t[so + idx], so uniform
 __device__ __forceinline__ float2 tab_at(const float2 *t, uint32_t so, uint32_t idx) {
@@ -524,43 +564,20 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
     const bool vec = ((A.lines | (uint32_t)((uintptr_t)A.out >> (DST == HH_F32 ? 2 : 1))) & 1u) == 0;
     auto put2 = [&](int32_t so, uint32_t vo, uint32_t l, float2 v) {
         constexpr int kUnit = DST == kDstPanels ? 8 : DST == HH_F32 ? 4 : 2;
-        glb8 *o = scalar_ptr(A.out, (int64_t)so * kUnit);
-        const uint32_t x = vo * kUnit;
-        if constexpr (DST == kDstPanels) {
-            st_s(o, x, f32x2{v.x, v.y});
-        } else if constexpr (DST == HH_F32) {
-            if (vec) {
-                st_s(o, x, f32x2{v.x, v.y});
-            } else {
-                st_s(o, x, v.x);
-                if (l + 1u < A.lines) st_s(o, x + 4u, v.y);
-            }
-        } else {
-            uint32_t b;
-            if constexpr (DST == HH_BF16) {
-                typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-                b = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v.x, (__bf16)v.y});
-            } else {
-                b = f32_to_f16_bits(v.x) | (f32_to_f16_bits(v.y) << 16);
-            }
-            if (vec) {
-                st_s(o, x, b);
-            } else {
-                st_s(o, x, (uint16_t)b);
-                if (l + 1u < A.lines) st_s(o, x + 2u, (uint16_t)(b >> 16));
-            }
-        }
+        store_pair<DST>(scalar_ptr(A.out, (int64_t)so * kUnit), vo, vec, l + 1u < A.lines, v);
     };
     // the output's steps: elements of a line, and where pair pr's lines are
-    const uint32_t ostep = DST == kDstPanels ? 1u << A.pcs : A.lines;
-    const int32_t obase = (int32_t)(DST == kDstPanels ? (grp * N) << A.pcs : line0);
+    const uint32_t osh = A.pcs + A.msh, part = (grp & ((1u << A.msh) - 1u)) << A.pcs;
+    const uint32_t ostep = DST == kDstPanels ? 1u << osh : A.lines;
+    const int32_t obase = (int32_t)(DST == kDstPanels ? (((grp >> A.msh) * N) << osh) + part : line0);
     auto opair = [&](uint32_t pr) -> uint32_t { return DST == kDstPanels ? pr : 2u * pr; };
 
     // (k, N - k) pairs, k = 0 with N / 2; a thread's are istep apart (a
     // multiple of 16, so LDS slots and panel offsets step linearly)
     const uint32_t nk = (N + 1u) / 2u, i0 = tid >> A.pcs, pr0 = tid & pm, istep = T >> A.pcs;
     const uint32_t sstep = (istep + (istep >> A.psh)) << A.pcs;
-    constexpr int CH = 4;  // of them loaded together
+    constexpr uint32_t kTasks = kPerThread / 2u;  // of them a thread, at most
+    constexpr uint32_t CH = 4;  // inverse: of them loaded together (4096^2 bf16 86 us; eight: 88)
     if constexpr (INV) {
         auto other = [&](uint32_t k) { return k == 0 ? N / 2u : N - k; };
         // Z[k] = s_1/2 w^k ((c1[k] + c2[N-k]) + i (c2[k] - c1[N-k])), w^(N-k) = i conj w^k,
@@ -752,7 +769,7 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
     auto store16 = [&](uint32_t i, uint32_t pr, const float2 (&x)[16]) {
         const uint32_t l = line0 + 2u * pr, nb = N / 16u;
         if constexpr (DST == kDstPanels) {
-            const uint32_t vv = (i << A.pcs) + pr;
+            const uint32_t vv = i * ostep + pr;
 #pragma unroll
             for (uint32_t j = 0; j < 16; j++) put2(obase + (int32_t)(j * nb * ostep), vv, l, x[j]);
         } else {
@@ -823,8 +840,13 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
         if (DST != kDstPanels && l >= A.lines) return;
         const uint32_t sk0 = slot(A, i0, pr0), sn0 = slot(A, N - i0, pr0);
         const uint32_t vk = i0 * ostep + opair(pr0), vn = (N - i0) * ostep + opair(pr0);
-        for (uint32_t c = 0; c * istep < nk; c++) {
-            if (i0 + c * istep >= nk) break;
+        float2 w[kTasks];
+#pragma unroll
+        for (uint32_t c = 0; c < kTasks; c++)
+            if (i0 + c * istep < nk) w[c] = tab_at(A.w4, c * istep, i0);
+#pragma unroll
+        for (uint32_t c = 0; c < kTasks; c++) {
+            if (i0 + c * istep >= nk) continue;
             const float2 zk = buf[sk0 + c * sstep];
             const int32_t so = (int32_t)(c * istep * ostep);
             if (c == 0 && i0 == 0) {
@@ -836,14 +858,58 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
                 }
             } else {
                 const float2 zn = buf[sn0 - c * sstep];
-                const float2 w = tab_at(A.w4, c * istep, i0);
                 const float r1 = zk.x + zn.x, i1 = zk.y - zn.y, r2 = zk.y + zn.y, i2 = zn.x - zk.x;
-                put2(obase + so, vk, l,
-                     make_float2(__builtin_fmaf(w.x, r1, w.y * i1), __builtin_fmaf(w.x, r2, w.y * i2)));
-                put2(obase - so, vn, l,
-                     make_float2(__builtin_fmaf(w.y, r1, -(w.x * i1)), __builtin_fmaf(w.y, r2, -(w.x * i2))));
+                put2(obase + so, vk, l, make_float2(__builtin_fmaf(w[c].x, r1, w[c].y * i1),
+                                                    __builtin_fmaf(w[c].x, r2, w[c].y * i2)));
+                put2(obase - so, vn, l, make_float2(__builtin_fmaf(w[c].y, r1, -(w[c].x * i1)),
+                                                    __builtin_fmaf(w[c].y, r2, -(w[c].x * i2))));
             }
         }
+    }
+}
+
+// The columns' panels (groups of 2 << pcs columns, N points each) to the
+// row-major result: 64 points of 64 columns per workgroup through LDS, rows
+// of 256 or 128 bytes out.  Bound by memory: 14336 x 4096 f32 81 us, 5.8 TB/s
+// (the device copy reaches 6.3).
+constexpr uint32_t kTileSide = 64, kTileStride = kTileSide + 2;  // even: pairs of columns stay aligned
+template <bool INV, int DST>
+__global__ __launch_bounds__(256) void untangle_kernel(Untangle U) {
+    __shared__ __attribute__((aligned(8))) float tile[kTileSide * kTileStride];
+    const uint32_t tid = threadIdx.x, t0 = blockIdx.x * kTileSide, c0 = blockIdx.y * kTileSide;
+    const uint32_t pm = (1u << U.pcs) - 1u, pairs = (U.lines + 1u) >> 1;
+    constexpr uint32_t kLoads = kTileSide * kTileSide / 2u / 256u;
+    f32x2 v[kLoads];
+    // 64 points of a group's pairs are contiguous (past the last: the last)
+    auto at = [&](uint32_t j, uint32_t &t, uint32_t &pr) {
+        const uint32_t e = tid + j * 256u, x = e & ((kTileSide << U.pcs) - 1u);
+        pr = ((e >> (6u + U.pcs)) << U.pcs) + (x & pm);
+        t = x >> U.pcs;
+    };
+#pragma unroll
+    for (uint32_t j = 0; j < kLoads; j++) {
+        uint32_t t, pr;
+        at(j, t, pr);
+        const uint32_t pair = c0 / 2u + pr < pairs ? c0 / 2u + pr : pairs - 1u, n = t0 + t < U.N ? t0 + t : U.N - 1u;
+        v[j] = *(const f32x2 *)(U.in + 2ull * ((((uint64_t)(pair >> U.pcs) * U.N + n) << U.pcs) + (pair & pm)));
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kLoads; j++) {
+        uint32_t t, pr;
+        at(j, t, pr);
+        *reinterpret_cast<f32x2 *>(&tile[t * kTileStride + 2u * pr]) = v[j];
+    }
+    __syncthreads();
+    const uint32_t c = (tid & 31u) * 2u, l = c0 + c;
+    if (l >= U.lines) return;
+    const bool vec = ((U.lines | (uint32_t)((uintptr_t)U.out >> (DST == HH_F32 ? 2 : 1))) & 1u) == 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kTileSide / 8u; j++) {
+        const uint32_t t = (tid >> 5) + j * 8u;
+        if (t0 + t >= U.N) break;
+        const f32x2 r = *reinterpret_cast<const f32x2 *>(&tile[t * kTileStride + c]);
+        const uint64_t o = (uint64_t)(INV ? element_of(t0 + t, U.N) : t0 + t) * U.lines + l;
+        store_pair<DST>(global(U.out), o, vec, l + 1u < U.lines, make_float2(r.x, r.y));
     }
 }
 
@@ -1005,6 +1071,7 @@ void fill(Lines &A, const LinePlan &P, const Split &S, uint32_t lines, const flo
     A.pcs = S.pcs;
     A.psh = P.psh;
     A.per_xcd = 0;
+    A.msh = 0;
     A.nr = P.nr;
     A.radix[0] = A.radix[1] = 0;
     for (uint32_t q = 0; q < P.nr; q++) A.radix[q >> 3] |= (uint64_t)P.r[q] << (8u * (q & 7u));
@@ -1021,8 +1088,39 @@ hipError_t launch_lines(const Lines &A, const Split &S, uint32_t grid, hipStream
     return hipGetLastError();
 }
 
+// Whether the columns go to the result by way of panels of their own and
+// untangle_kernel.  A workgroup of two columns (more than 8192 rows) writes 8
+// or 4 bytes of a row: 14336 x 4096 forward 394 us for that pass, against 241
+// to panels and 81 for the tiles; inverse, whole, 489 -> 450 (bf16 437 -> 424).
+// Four columns gain nothing (8192 x 4096 232 -> 265), nor do lengths with a
+// prime pass, whose workgroups don't write all at once (11008 x 4096 bf16 498
+// -> 523).
+bool through_panels(const LinePlan &Ph) { return Ph.N > kMaxPoints / 2u && Ph.roots == 0; }
+
+// log2 of the row workgroups that share a panel.  A column workgroup reads
+// pieces of 2 PC columns x G rows; below a line of memory (128 bytes) two
+// share: 4096 x 14336 bf16 375 -> 353 us, 8192^2 459 -> 437 (four: 378, 479).
+// Before untangle_kernel 256 bytes pay, four at most: 14336 x 4096 485 -> 458
+// (two) -> 445 us, 12288 x 3072 334 -> 301 -> 293; eight no more.
+uint32_t panel_share(const LinePlan &Pw, const LinePlan &Ph, const Split &Sw, const Split &Sh) {
+    const bool through = through_panels(Ph);
+    const uint32_t piece = 4u + Sw.pcs + Sh.pcs, want = through ? 8u : 7u, most = through ? 2u : 1u;
+    return piece >= want ? 0u : want - piece < most ? want - piece : most;
+}
+
+// The f32 panels of the rows (whole panels) and those of the columns.
+size_t row_panels(const LinePlan &Pw, const LinePlan &Ph, const Split &Sw, const Split &Sh) {
+    const uint32_t g = 2u << (Sw.pcs + panel_share(Pw, Ph, Sw, Sh));
+    return (size_t)((Ph.N + g - 1u) / g * g) * Pw.N;
+}
+size_t panel_elems(const LinePlan &Pw, const LinePlan &Ph, const Split &Sw, const Split &Sh) {
+    const uint32_t g = 2u << Sh.pcs;
+    return row_panels(Pw, Ph, Sw, Sh) + (through_panels(Ph) ? (size_t)((Pw.N + g - 1u) / g * g) * Ph.N : 0u);
+}
+
 // Both passes of an h x w transform: rows (from d_in, or the fragments in F)
-// to panels in d_mid, columns to d_out.
+// to panels in d_mid, columns to d_out, where they don't lie a line of memory
+// side by side by way of panels and tiles.
 int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines *F, float *d_mid, const LinePlan &Pw,
                    const LinePlan &Ph, const Split &Sw, const Split &Sh, int32_t dtype, void *d_out, hipStream_t s) {
     const float2 *tw, *th;
@@ -1038,7 +1136,12 @@ int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines
     A.coef_f32 = cf;
     A.in = d_in;
     A.out = d_mid;
-    const uint32_t ga = (h + (2u << Sw.pcs) - 1u) >> (Sw.pcs + 1u);
+    uint32_t ga = (h + (2u << Sw.pcs) - 1u) >> (Sw.pcs + 1u);
+    A.msh = panel_share(Pw, Ph, Sw, Sh);
+    if (A.msh) {
+        A.per_xcd = (((ga + 7u) / 8u - 1u) | ((1u << A.msh) - 1u)) + 1u;
+        ga = 8u * A.per_xcd;
+    }
     hipError_t e = F         ? launch_lines<true, kSrcFrags, kDstPanels>(A, Sw, ga, s)
                    : inverse ? launch_lines<true, kSrcRows, kDstPanels>(A, Sw, ga, s)
                              : launch_lines<false, kSrcRows, kDstPanels>(A, Sw, ga, s);
@@ -1047,19 +1150,37 @@ int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines
     fill(B, Ph, Sh, w, th);
     B.in = d_mid;
     B.out = d_out;
-    B.gsh = Sw.pcs + 1u;
+    B.gsh = Sw.pcs + A.msh + 1u;
     const uint32_t gb = (w + (2u << Sh.pcs) - 1u) >> (Sh.pcs + 1u);
     B.per_xcd = (gb + 7u) / 8u;
     const uint32_t grid = 8u * B.per_xcd;
+    if (!through_panels(Ph)) {
+        if (!inverse)
+            e = launch_lines<false, kSrcPanels, HH_F32>(B, Sh, grid, s);
+        else if (dtype == HH_BF16)
+            e = launch_lines<true, kSrcPanels, HH_BF16>(B, Sh, grid, s);
+        else if (dtype == HH_F16)
+            e = launch_lines<true, kSrcPanels, HH_F16>(B, Sh, grid, s);
+        else
+            e = launch_lines<true, kSrcPanels, HH_F32>(B, Sh, grid, s);
+        return from_hip(e);
+    }
+    float *cols = d_mid + row_panels(Pw, Ph, Sw, Sh);
+    B.out = cols;
+    e = inverse ? launch_lines<true, kSrcPanels, kDstPanels>(B, Sh, grid, s)
+                : launch_lines<false, kSrcPanels, kDstPanels>(B, Sh, grid, s);
+    if (e != hipSuccess) return from_hip(e);
+    const Untangle U{cols, d_out, h, w, Sh.pcs};
+    const dim3 tiles((h + kTileSide - 1u) / kTileSide, (w + kTileSide - 1u) / kTileSide);
     if (!inverse)
-        e = launch_lines<false, kSrcPanels, HH_F32>(B, Sh, grid, s);
+        hipLaunchKernelGGL((untangle_kernel<false, HH_F32>), tiles, dim3(256), 0, s, U);
     else if (dtype == HH_BF16)
-        e = launch_lines<true, kSrcPanels, HH_BF16>(B, Sh, grid, s);
+        hipLaunchKernelGGL((untangle_kernel<true, HH_BF16>), tiles, dim3(256), 0, s, U);
     else if (dtype == HH_F16)
-        e = launch_lines<true, kSrcPanels, HH_F16>(B, Sh, grid, s);
+        hipLaunchKernelGGL((untangle_kernel<true, HH_F16>), tiles, dim3(256), 0, s, U);
     else
-        e = launch_lines<true, kSrcPanels, HH_F32>(B, Sh, grid, s);
-    return from_hip(e);
+        hipLaunchKernelGGL((untangle_kernel<true, HH_F32>), tiles, dim3(256), 0, s, U);
+    return from_hip(hipGetLastError());
 }
 
 bool make_plans(const hh_context *ctx, uint32_t h, uint32_t w, bool frags, LinePlan &Pw, LinePlan &Ph, Split &Sw,
@@ -1067,12 +1188,6 @@ bool make_plans(const hh_context *ctx, uint32_t h, uint32_t w, bool frags, LineP
     const uint32_t want = ctx->num_cus > 0 ? (uint32_t)ctx->num_cus : 256u;
     return make_line_plan(w, Pw) && make_line_plan(h, Ph) && make_split(Pw, h, frags, want, Sw) &&
            make_split(Ph, w, false, want, Sh);
-}
-
-// The f32 panels (whole panels of 2 PC rows).
-size_t mid_elems(uint32_t h, uint32_t w, const Split &Sw) {
-    const uint32_t g = 2u << Sw.pcs;
-    return (size_t)((h + g - 1u) / g * g) * w;
 }
 
 int32_t mid_scratch(hh_context *ctx, size_t bytes, hipStream_t s, uint8_t **out) {
@@ -1109,7 +1224,7 @@ int32_t dct2d_lines(hh_context *ctx, bool inverse, const float *d_in, uint32_t h
     Split Sw, Sh;
     if (!make_plans(ctx, h, w, false, Pw, Ph, Sw, Sh)) return HH_ERR_UNSUPPORTED;
     uint8_t *mid;
-    int32_t rc = mid_scratch(ctx, mid_elems(h, w, Sw) * sizeof(float), s, &mid);
+    int32_t rc = mid_scratch(ctx, panel_elems(Pw, Ph, Sw, Sh) * sizeof(float), s, &mid);
     if (rc != HH_OK) return rc;
     return two_passes(ctx, inverse, d_in, nullptr, reinterpret_cast<float *>(mid), Pw, Ph, Sw, Sh, out_dtype, d_out, s);
 }
@@ -1119,7 +1234,7 @@ int32_t hct3_decode_lines(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrag
     LinePlan Pw, Ph;
     Split Sw, Sh;
     if (nfrags == 0 || nfrags > kMaxFrags || !make_plans(ctx, h, w, true, Pw, Ph, Sw, Sh)) return HH_ERR_UNSUPPORTED;
-    const size_t mid_bytes = (mid_elems(h, w, Sw) * sizeof(float) + 255u) & ~(size_t)255u;
+    const size_t mid_bytes = (panel_elems(Pw, Ph, Sw, Sh) * sizeof(float) + 255u) & ~(size_t)255u;
     uint8_t *mid;
     int32_t rc = mid_scratch(ctx, mid_bytes + (size_t)nfrags * h * 4u, s, &mid);
     if (rc != HH_OK) return rc;

@@ -1,8 +1,10 @@
 """The two-pass whole-matrix transforms (csrc/dct_lines.hip) at the lengths
 where they can go wrong: one line, odd numbers of lines and lengths, every
 radix and the direct sums of the other primes, padded and unpadded LDS
-layouts, the longest lines, outputs that are not aligned; and HCT3 fragments
-whose rows start inside a bitmap byte.
+layouts, the longest lines, columns that go to the result by way of panels
+(more than 8192 rows) with ragged tiles, panels that several workgroups share,
+outputs that are not aligned; and HCT3 fragments whose rows start inside a
+bitmap byte.
 
 Bound: a length-N f32 FFT has a relative 2-norm error of about
 0.6 eps sqrt(log2 N) per pass (eps = 2^-24 roundings of the sums, as much
@@ -32,7 +34,8 @@ def basis64(n):
 
 @pytest.mark.parametrize("rows,cols", [(1, 1), (1, 77), (2, 3), (16, 17), (37, 53), (127, 126), (143, 11), (48, 80),
                                        (320, 448), (576, 576), (640, 1376), (2752, 96), (255, 1000), (16384, 34),
-                                       (33, 16384), (11008, 64), (64, 14336), (4096, 66)])
+                                       (33, 16384), (11008, 64), (64, 14336), (4096, 66), (8505, 5), (8232, 64),
+                                       (9000, 67), (16384, 129), (12288, 1025), (301, 9000)])
 def test_transforms_vs_f64(rows, cols):
     T, h, c = G.torch(), H(), G.ctx()
     x = T.randn(rows, cols, device="cuda", generator=T.Generator(device="cuda").manual_seed(rows + cols))
