@@ -140,7 +140,7 @@ bool zstd_framed(const uint8_t *d, size_t len) {
 // GpuDecompressor::try_zstd_decompress (decompress.rs:296-319): zstd-framed
 // input is decoded on the host; if that fails the bytes are parsed as a raw
 // container.  Returns whether `hold` now holds the decoded container.
-bool unwrap_zstd(const uint8_t *&data, size_t &len, std::vector<uint8_t> &hold) {
+bool unwrap_zstd(const uint8_t *&data, size_t &len, hh::HostBytes &hold) {
     if (!zstd_framed(data, len) || !hh::zstd_decode_all(data, len, hold)) return false;
     data = hold.data();
     len = hold.size();
@@ -225,6 +225,200 @@ int32_t decode_eo(hh_context *ctx, const std::vector<Layer> &layers, const uint8
     return hh::hct3_decode_eo(ctx, fr.data(), (uint32_t)fr.size(), rows, cols, dtype, d_out, d_stage, s);
 }
 
+// A spectral tensor's fragments, parsed: fragment 0's bitmap and where the
+// coefficients (index-map order, csz bytes each) come from.
+struct Spectral {
+    struct Piece {
+        size_t at, bytes;  // in the coefficients
+        const uint8_t *src;
+    };
+    const uint8_t *bitmap = nullptr;
+    uint64_t bm = 0, n = 0;
+    uint32_t w = 0, h = 0, ntot = 0;
+    int f32c = 0;
+    bool sized = false;  // w and h are set
+    std::vector<Piece> pieces;
+    size_t coef_bytes() const { return (size_t)ntot * (f32c ? 4 : 2); }
+    // every coefficient comes from some piece, none from before its turn
+    bool whole() const {
+        size_t end = 0;
+        for (const Piece &p : pieces) {
+            if (p.at > end) return false;
+            end = std::max(end, p.at + p.bytes);
+        }
+        return end == coef_bytes();
+    }
+    // few enough copies of their own, and nothing between them to clear
+    bool pieces_fit() const { return pieces.size() <= 16 && whole(); }
+    void assemble(uint8_t *coef) const {
+        if (!whole()) std::memset(coef, 0, coef_bytes());  // unset entries stay 0.0
+        for (const Piece &p : pieces) std::memcpy(coef + p.at, p.src, p.bytes);
+    }
+};
+
+// Set bits of n bytes; popcount_hw by the processor's own instruction, for
+// whole 32 bytes (480 kB 21 against 48 us).
+__attribute__((target("popcnt"))) uint64_t popcount_hw(const uint8_t *p, size_t n) {
+    uint64_t c[4] = {0, 0, 0, 0};
+    for (size_t i = 0; i + 32 <= n; i += 32) {
+        uint64_t w[4];
+        std::memcpy(w, p + i, 32);
+        for (int j = 0; j < 4; j++) c[j] += (uint64_t)__builtin_popcountll(w[j]);
+    }
+    return c[0] + c[1] + c[2] + c[3];
+}
+uint64_t popcount(const uint8_t *p, size_t n) {
+    size_t i = 0;
+    uint64_t c = 0;
+    if (__builtin_cpu_supports("popcnt")) {
+        i = n & ~(size_t)31;
+        c = popcount_hw(p, i);
+    }
+    for (; i + 8 <= n; i += 8) {
+        uint64_t w;
+        std::memcpy(&w, p + i, 8);
+        c += (uint64_t)__builtin_popcountll(w);
+    }
+    for (; i < n; i++) c += (uint64_t)__builtin_popcount((uint32_t)p[i]);
+    return c;
+}
+
+// The checks of add_essentials and add_detail (compressive.rs:438-465,
+// :653-700).
+int32_t spectral_parse(const uint8_t *const *frags, const size_t *frag_lens, const uint16_t *frag_index,
+                       uint32_t nfrags, Spectral &S, hh_block_status *status) {
+    auto corrupt = [&](int32_t detail) {
+        if (status) {
+            status->code = HH_ERR_CORRUPTED_DATA;
+            status->detail = detail;
+        }
+        return (int32_t)HH_ERR_CORRUPTED_DATA;
+    };
+    if (frag_index[0] != 0) return corrupt(HH_CORRUPT_HEADER);  // "fragment 0 must be added first"
+    const uint8_t *f0 = frags[0];
+    const size_t l0 = frag_lens[0];
+    if (!f0 || l0 < 24) return corrupt(HH_CORRUPT_SIZE);  // "fragment 0 too short"
+    const uint32_t magic = rd32(f0);
+    // V1 (explicit index array, compressive.rs:467-520) is not decoded here
+    if (magic != kMagicHct3 && magic != kMagicHct2) return HH_ERR_UNSUPPORTED;
+    S.f32c = magic == kMagicHct2;
+    const size_t csz = S.f32c ? 4 : 2;
+    const uint32_t ntot = rd32(f0 + 12), ness = rd32(f0 + 16), dpf = rd32(f0 + 20);
+    S.w = rd32(f0 + 4);
+    S.h = rd32(f0 + 8);
+    S.sized = true;
+    S.ntot = ntot;
+    S.n = (uint64_t)S.w * S.h;
+    if (S.n > 0xffffffffull || S.w > 0x7fffffffu || S.h > 0x7fffffffu) return HH_ERR_INVALID_ARGUMENT;
+    S.bm = (S.n + 7) / 8;
+    if (24 + S.bm > l0) return corrupt(HH_CORRUPT_SIZE);  // "truncated bitmap"
+    S.bitmap = f0 + 24;
+    uint64_t cnt = popcount(S.bitmap, (size_t)S.bm);
+    if (S.n & 7)
+        cnt -= (uint64_t)__builtin_popcount((uint32_t)S.bitmap[S.bm - 1] & ~((1u << (S.n & 7)) - 1) & 0xffu);
+    if (cnt != ntot) return corrupt(HH_CORRUPT_BITMAP_COUNT);  // compressive.rs:630-636
+    // coefficients in index-map order
+    const size_t off = 24 + (size_t)S.bm;
+    // "truncated essential coefficients", or more of them than retained
+    // positions (the reference indexes past its array): both a size error
+    if ((uint64_t)ness * csz > l0 - off || ness > ntot) return corrupt(HH_CORRUPT_SIZE);
+    if (ness) S.pieces.push_back({0, (size_t)ness * csz, f0 + off});
+    for (uint32_t f = 1; f < nfrags; f++) {
+        if (frag_index[f] == 0) continue;
+        const uint8_t *d = frags[f];
+        const size_t l = frag_lens[f];
+        if (!d || l < 8) return corrupt(HH_CORRUPT_SIZE);  // "detail fragment too short"
+        const uint32_t fi = rd16(d);
+        const uint32_t count = rd32(d + 4);
+        if (fi == 0) return corrupt(HH_CORRUPT_HEADER);  // start would underflow in the reference
+        const uint64_t start = (uint64_t)ness + (uint64_t)(fi - 1) * dpf;
+        // the values present (up to count), those at positions below ntot
+        uint64_t nv = (l - 8) / csz;
+        if (nv > count) nv = count;
+        if (start < ntot) {
+            const uint64_t m = nv < ntot - start ? nv : ntot - start;
+            if (m) S.pieces.push_back({(size_t)start * csz, (size_t)m * csz, d + 8});
+        }
+    }
+    return HH_OK;
+}
+
+int32_t spectral_output(const Spectral &S, const void *d_out, uint64_t out_cap, hh_block_status *status) {
+    if (!d_out) return HH_ERR_INVALID_ARGUMENT;
+    if (out_cap >= S.n) return HH_OK;
+    if (status) {
+        status->code = HH_ERR_BUFFER_TOO_SMALL;
+        status->required = S.n;
+    }
+    return HH_ERR_BUFFER_TOO_SMALL;
+}
+
+bool spectral_lines(const hh_context *ctx, const Spectral &S) {
+    return lines_candidate(ctx, {Layer{S.bitmap, nullptr, S.ntot}}, S.h, S.w);
+}
+
+// Bitmap and coefficients to the context's scratch: from where they lie if
+// that is pinned memory (the staging buffer), else put together there, or in
+// ordinary memory if they don't fit.  `own` keeps that until the copies are
+// done; the caller waits for them.
+int32_t spectral_upload(hh_context *ctx, const Spectral &S, bool pinned, hipStream_t s,
+                        std::vector<uint8_t> *own = nullptr) {
+    const size_t words = align16((size_t)S.bm), cb = S.coef_bytes();
+    int32_t rc = ensure_scratch(ctx, words + align16(cb));
+    if (rc != HH_OK) return rc;
+    uint8_t *d_bits = reinterpret_cast<uint8_t *>(ctx->d_scratch), *d_coef = d_bits + words;
+    hipError_t e;
+    if (pinned && S.pieces_fit()) {
+        e = hipMemcpyAsync(d_bits, S.bitmap, (size_t)S.bm, hipMemcpyHostToDevice, s);
+        for (const Spectral::Piece &p : S.pieces)
+            if (e == hipSuccess) e = hipMemcpyAsync(d_coef + p.at, p.src, p.bytes, hipMemcpyHostToDevice, s);
+        return from_hip(e);
+    }
+    uint8_t *h = pinned ? nullptr : hh::host_stage(ctx, words + cb, 0);
+    if (!h) {
+        own->resize(words + cb);
+        h = own->data();
+    }
+    std::memcpy(h, S.bitmap, (size_t)S.bm);
+    S.assemble(h + words);
+    return from_hip(hipMemcpyAsync(d_bits, h, words + cb, hipMemcpyHostToDevice, s));
+}
+
+// reconstruct (compressive.rs:728-752): one scatter with fragment 0's bitmap.
+// pinned: the fragments lie in the staging buffer; uploaded: spectral_upload
+// has run.
+int32_t spectral_decode(hh_context *ctx, const Spectral &S, bool pinned, bool uploaded, int32_t out_dtype,
+                        void *d_out, hh_block_status *status, hipStream_t s) {
+    std::vector<uint8_t> own;
+    if (spectral_lines(ctx, S)) {
+        int32_t rc = uploaded ? (int32_t)HH_OK : spectral_upload(ctx, S, pinned, s, &own);
+        if (rc == HH_OK) {
+            uint8_t *d_bits = reinterpret_cast<uint8_t *>(ctx->d_scratch);
+            const hh::Hct3Frag F{d_bits, d_bits + align16((size_t)S.bm), S.ntot};
+            rc = hh::hct3_decode_lines(ctx, &F, 1, S.f32c != 0, S.h, S.w, out_dtype, d_out, s);
+        }
+        const hipError_t e = hipStreamSynchronize(s);  // also after an error: the staging buffer is free again
+        if (rc == HH_OK) rc = from_hip(e);
+        if (rc == HH_OK && status) status->written = S.n;
+        return rc;
+    }
+    own.resize(S.coef_bytes());
+    S.assemble(own.data());
+    std::vector<Layer> layers{Layer{S.bitmap, own.data(), S.ntot}};
+    const size_t mat = align16((size_t)S.n * sizeof(float));
+    int32_t rc = ensure_scratch(ctx, 2 * mat + stage_bytes(S.n, S.ntot, S.f32c));
+    if (rc != HH_OK) return rc;
+    uint8_t *base = reinterpret_cast<uint8_t *>(ctx->d_scratch);
+    float *d_dense = reinterpret_cast<float *>(base);
+    float *d_tmp = reinterpret_cast<float *>(base + mat);
+    rc = scatter_layers(layers, S.n, S.f32c, d_dense, base + 2 * mat, s);
+    if (rc == HH_OK) rc = inverse_to(ctx, d_dense, d_tmp, S.h, S.w, out_dtype, d_out, s, !S.f32c);
+    const hipError_t e = hipStreamSynchronize(s);
+    if (rc == HH_OK) rc = from_hip(e);
+    if (rc == HH_OK && status) status->written = S.n;
+    return rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -232,7 +426,7 @@ extern "C" {
 int32_t hh_hct3_coefficients(hh_context *ctx, const uint8_t *data, size_t len, uint64_t total,
                              float *d_coeffs, void *stream) {
     if (!ctx || !data || (total && !d_coeffs) || total > 0xffffffffull) return HH_ERR_INVALID_ARGUMENT;
-    std::vector<uint8_t> hold;
+    hh::HostBytes hold;
     unwrap_zstd(data, len, hold);
     std::vector<Layer> layers;
     int32_t rc = parse_container(data, len, total, layers);
@@ -256,7 +450,7 @@ int32_t hh_hct3_decompress(hh_context *ctx, const uint8_t *data, size_t len, con
     uint32_t rows, cols;
     int32_t rc = dims_of(shape, rank, &total, &rows, &cols);
     if (rc != HH_OK) return rc;
-    std::vector<uint8_t> hold;
+    hh::HostBytes hold;
     unwrap_zstd(data, len, hold);
     std::vector<Layer> layers;
     rc = parse_container(data, len, total, layers);
@@ -347,110 +541,18 @@ int32_t hh_spectral_reconstruct(hh_context *ctx, const uint8_t *const *frags, co
                                 void *d_out, uint64_t out_cap, uint32_t *width, uint32_t *height,
                                 hh_block_status *status, void *stream) {
     if (status) std::memset(status, 0, sizeof(*status));
-    auto corrupt = [&](int32_t detail) {
-        if (status) {
-            status->code = HH_ERR_CORRUPTED_DATA;
-            status->detail = detail;
-        }
-        return (int32_t)HH_ERR_CORRUPTED_DATA;
-    };
     if (!ctx || !frags || !frag_lens || !frag_index || nfrags == 0 || !valid_dtype(out_dtype))
         return HH_ERR_INVALID_ARGUMENT;
-    // add_essentials (compressive.rs:438-465)
-    if (frag_index[0] != 0) return corrupt(HH_CORRUPT_HEADER);  // "fragment 0 must be added first"
-    const uint8_t *f0 = frags[0];
-    const size_t l0 = frag_lens[0];
-    if (!f0 || l0 < 24) return corrupt(HH_CORRUPT_SIZE);  // "fragment 0 too short"
-    const uint32_t magic = rd32(f0);
-    // V1 (explicit index array, compressive.rs:467-520) is not decoded here
-    if (magic != kMagicHct3 && magic != kMagicHct2) return HH_ERR_UNSUPPORTED;
-    const int f32c = magic == kMagicHct2;
-    const size_t csz = f32c ? 4 : 2;
-    const uint32_t w = rd32(f0 + 4), h = rd32(f0 + 8), ntot = rd32(f0 + 12), ness = rd32(f0 + 16),
-                   dpf = rd32(f0 + 20);
-    const uint64_t n = (uint64_t)w * h;
-    if (width) *width = w;
-    if (height) *height = h;
-    if (n > 0xffffffffull || w > 0x7fffffffu || h > 0x7fffffffu) return HH_ERR_INVALID_ARGUMENT;
-    const uint64_t bm = (n + 7) / 8;
-    if (24 + bm > l0) return corrupt(HH_CORRUPT_SIZE);  // "truncated bitmap"
-    uint64_t cnt = 0;
-    {
-        const uint8_t *bp = f0 + 24;
-        uint64_t i = 0;
-        for (; i + 8 <= bm; i += 8) {
-            uint64_t wv;
-            std::memcpy(&wv, bp + i, 8);
-            cnt += (uint64_t)__builtin_popcountll(wv);
-        }
-        for (; i < bm; i++) cnt += (uint64_t)__builtin_popcount((uint32_t)bp[i]);
-        if (n & 7) cnt -= (uint64_t)__builtin_popcount((uint32_t)bp[bm - 1] & ~((1u << (n & 7)) - 1) & 0xffu);
-    }
-    if (cnt != ntot) return corrupt(HH_CORRUPT_BITMAP_COUNT);  // compressive.rs:630-636
-    // coefficients in index-map order; unset entries stay 0.0
-    std::vector<uint8_t> coef((size_t)ntot * csz, 0);
-    const size_t off = 24 + (size_t)bm;
-    // "truncated essential coefficients", or more of them than retained
-    // positions (the reference indexes past its array): both a size error
-    if ((uint64_t)ness * csz > l0 - off || ness > ntot) return corrupt(HH_CORRUPT_SIZE);
-    if (ness) std::memcpy(coef.data(), f0 + off, (size_t)ness * csz);
-    // add_detail (compressive.rs:653-700)
-    for (uint32_t f = 1; f < nfrags; f++) {
-        if (frag_index[f] == 0) continue;
-        const uint8_t *d = frags[f];
-        const size_t l = frag_lens[f];
-        if (!d || l < 8) return corrupt(HH_CORRUPT_SIZE);  // "detail fragment too short"
-        const uint32_t fi = rd16(d);
-        const uint32_t count = rd32(d + 4);
-        if (fi == 0) return corrupt(HH_CORRUPT_HEADER);  // start would underflow in the reference
-        const uint64_t start = (uint64_t)ness + (uint64_t)(fi - 1) * dpf;
-        // the values present (up to count), those at positions below ntot
-        uint64_t nv = (l - 8) / csz;
-        if (nv > count) nv = count;
-        if (start < ntot) {
-            const uint64_t m = nv < ntot - start ? nv : ntot - start;
-            if (m) std::memcpy(&coef[(size_t)start * csz], d + 8, (size_t)m * csz);
-        }
-    }
-    if (n == 0) return HH_OK;
-    if (!d_out) return HH_ERR_INVALID_ARGUMENT;
-    if (out_cap < n) {
-        if (status) {
-            status->code = HH_ERR_BUFFER_TOO_SMALL;
-            status->required = n;
-        }
-        return HH_ERR_BUFFER_TOO_SMALL;
-    }
-    // reconstruct (compressive.rs:728-752): one scatter with fragment 0's bitmap
+    Spectral S;
+    int32_t rc = spectral_parse(frags, frag_lens, frag_index, nfrags, S, status);
+    if (S.sized && width) *width = S.w;
+    if (S.sized && height) *height = S.h;
+    if (rc != HH_OK || S.n == 0) return rc;
+    rc = spectral_output(S, d_out, out_cap, status);
+    if (rc != HH_OK) return rc;
     hh::DeviceGuard guard(ctx->device);
     if (guard.status() != hipSuccess) return from_hip(guard.status());
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    std::vector<Layer> layers{Layer{f0 + 24, coef.data(), ntot}};
-    if (lines_candidate(ctx, layers, h, w)) {
-        const size_t words = align16((size_t)bm);
-        int32_t rc = ensure_scratch(ctx, words + align16(coef.size()));
-        if (rc != HH_OK) return rc;
-        uint8_t *d_bits = reinterpret_cast<uint8_t *>(ctx->d_scratch), *d_coef = d_bits + words;
-        hipError_t e = hipMemcpyAsync(d_bits, f0 + 24, (size_t)bm, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess && ntot) e = hipMemcpyAsync(d_coef, coef.data(), coef.size(), hipMemcpyHostToDevice, s);
-        if (e != hipSuccess) return from_hip(e);
-        const hh::Hct3Frag F{d_bits, d_coef, ntot};
-        rc = hh::hct3_decode_lines(ctx, &F, 1, f32c != 0, h, w, out_dtype, d_out, s);
-        if (rc != HH_OK) return rc;
-        if (status) status->written = n;
-        return from_hip(hipStreamSynchronize(s));
-    }
-    const size_t mat = align16((size_t)n * sizeof(float));
-    int32_t rc = ensure_scratch(ctx, 2 * mat + stage_bytes(n, ntot, f32c));
-    if (rc != HH_OK) return rc;
-    uint8_t *base = reinterpret_cast<uint8_t *>(ctx->d_scratch);
-    float *d_dense = reinterpret_cast<float *>(base);
-    float *d_tmp = reinterpret_cast<float *>(base + mat);
-    rc = scatter_layers(layers, n, f32c, d_dense, base + 2 * mat, s);
-    if (rc == HH_OK) rc = inverse_to(ctx, d_dense, d_tmp, h, w, out_dtype, d_out, s, !f32c);
-    if (rc != HH_OK) return rc;
-    if (status) status->written = n;
-    return from_hip(hipStreamSynchronize(s));
+    return spectral_decode(ctx, S, false, false, out_dtype, d_out, status, reinterpret_cast<hipStream_t>(stream));
 }
 
 int32_t hh_turbo_tensor_decode(hh_context *ctx, const uint8_t *data, size_t len, int32_t verify,
@@ -458,8 +560,18 @@ int32_t hh_turbo_tensor_decode(hh_context *ctx, const uint8_t *data, size_t len,
                                uint32_t *height, hh_block_status *status, void *stream) {
     if (status) std::memset(status, 0, sizeof(*status));
     if (!ctx || !data) return HH_ERR_INVALID_ARGUMENT;
-    // zstd wrapper (turbo.rs:389-391); the container inside (:378-387)
-    std::vector<uint8_t> hold;
+    hh::DeviceGuard guard(ctx->device);
+    if (guard.status() != hipSuccess) return from_hip(guard.status());
+    // zstd wrapper (turbo.rs:389-391), decoded into the pinned staging buffer
+    // while that has room; the container inside (:378-387)
+    hh::HostBytes hold(
+        [](void *owner, size_t bytes, size_t *cap) {
+            hh_context *c = static_cast<hh_context *>(owner);
+            uint8_t *p = hh::host_stage(c, bytes, c->stage_bytes);
+            *cap = c->stage_bytes;
+            return p;
+        },
+        ctx);
     if (zstd_framed(data, len)) {
         if (!hh::zstd_decode_all(data, len, hold)) {
             if (status) status->code = HH_ERR_CORRUPTED_DATA;
@@ -468,6 +580,7 @@ int32_t hh_turbo_tensor_decode(hh_context *ctx, const uint8_t *data, size_t len,
         data = hold.data();
         len = hold.size();
     }
+    const bool pinned = hold.size() > 0 && !hold.owned();
     auto bad = [&](int32_t detail) {
         if (status) {
             status->code = HH_ERR_CORRUPTED_DATA;
@@ -480,39 +593,77 @@ int32_t hh_turbo_tensor_decode(hh_context *ctx, const uint8_t *data, size_t len,
     std::vector<const uint8_t *> ptrs;
     std::vector<size_t> lens;
     std::vector<uint16_t> idx;
+    std::vector<uint64_t> sums;
     size_t off = 2;
-    for (uint32_t f = 0; f < nf; f++) {
-        if (len - off < 16) return bad(HH_CORRUPT_SIZE);
+    bool truncated = false;
+    for (uint32_t f = 0; f < nf && !truncated; f++) {
+        truncated = len - off < 16;
+        if (truncated) break;
         const uint16_t fi = rd16(data + off);
         uint64_t sum = 0;
         for (int i = 0; i < 8; i++) sum |= (uint64_t)data[off + 4 + i] << (8 * i);
         const uint32_t dl = rd32(data + off + 12);
         off += 16;
-        if ((size_t)dl > len - off) return bad(HH_CORRUPT_SIZE);
-        // HoloFragment::new stores xxh3_64 of the fragment data (holotensor.rs:285)
-        if (verify && hh::xxh3_64_host(data + off, dl) != sum) {
-            if (status) {
-                status->code = HH_ERR_CHECKSUM_MISMATCH;
-                status->position = f;
-            }
-            return HH_ERR_CHECKSUM_MISMATCH;
-        }
+        truncated = (size_t)dl > len - off;
+        if (truncated) break;
         ptrs.push_back(data + off);
         lens.push_back(dl);
         idx.push_back(fi);
+        sums.push_back(sum);
         off += dl;
     }
-    if (nf == 0) return bad(HH_CORRUPT_HEADER);
+    // HoloFragment::new stores xxh3_64 of the fragment data
+    // (holotensor.rs:285): the first that differs, before the truncated one
+    auto check = [&]() -> int32_t {
+        for (size_t f = 0; verify && f < sums.size(); f++)
+            if (hh::xxh3_64_host(ptrs[f], lens[f]) != sums[f]) {
+                if (status) {
+                    status->code = HH_ERR_CHECKSUM_MISMATCH;
+                    status->position = f;
+                }
+                return HH_ERR_CHECKSUM_MISMATCH;
+            }
+        return HH_OK;
+    };
+    if (truncated || nf == 0) {
+        const int32_t rc = check();
+        return rc != HH_OK ? rc : bad(nf == 0 ? HH_CORRUPT_HEADER : HH_CORRUPT_SIZE);
+    }
     // fragment 0 (the essentials) goes in first, the details keep their order
+    std::vector<const uint8_t *> fp = ptrs;
+    std::vector<size_t> fl = lens;
     for (uint32_t f = 1; f < nf; f++)
         if (idx[f] == 0 && idx[0] != 0) {
-            std::rotate(ptrs.begin(), ptrs.begin() + f, ptrs.begin() + f + 1);
-            std::rotate(lens.begin(), lens.begin() + f, lens.begin() + f + 1);
+            std::rotate(fp.begin(), fp.begin() + f, fp.begin() + f + 1);
+            std::rotate(fl.begin(), fl.begin() + f, fl.begin() + f + 1);
             std::rotate(idx.begin(), idx.begin() + f, idx.begin() + f + 1);
             break;
         }
-    return hh_spectral_reconstruct(ctx, ptrs.data(), lens.data(), idx.data(), nf, out_dtype, d_out, out_cap,
-                                   width, height, status, stream);
+    // Everything is checked before the first kernel runs, but where nothing
+    // else is wrong the copies to the device's scratch run while the host
+    // verifies the checksums (2 MB: 76 us).
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    Spectral S;
+    hh_block_status st;
+    std::memset(&st, 0, sizeof(st));
+    int32_t rc = valid_dtype(out_dtype) ? spectral_parse(fp.data(), fl.data(), idx.data(), nf, S, &st)
+                                        : (int32_t)HH_ERR_INVALID_ARGUMENT;
+    if (rc == HH_OK && S.n) rc = spectral_output(S, d_out, out_cap, &st);
+    bool uploaded = false;
+    if (rc == HH_OK && S.n && pinned && spectral_lines(ctx, S) && S.pieces_fit()) {
+        rc = spectral_upload(ctx, S, true, s);
+        uploaded = true;
+    }
+    const int32_t sum_rc = check();
+    if (sum_rc != HH_OK || rc != HH_OK) {
+        if (uploaded) (void)hipStreamSynchronize(s);
+        if (sum_rc != HH_OK) return sum_rc;
+        if (status) *status = st;
+    }
+    if (S.sized && width) *width = S.w;
+    if (S.sized && height) *height = S.h;
+    if (rc != HH_OK || S.n == 0) return rc;
+    return spectral_decode(ctx, S, pinned, uploaded, out_dtype, d_out, status, s);
 }
 
 int32_t hh_idct_2d(hh_context *ctx, const float *d_in, uint32_t rows, uint32_t cols, int32_t out_dtype,

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/haagenti_hip.h"
+#include "host_bytes.hpp"
 
 struct hh_context {
     int device = 0;
@@ -19,6 +20,13 @@ struct hh_context {
     // (grown on demand, kept until the context is destroyed).
     void *d_scratch = nullptr;
     size_t scratch_bytes = 0;
+    // Pinned host memory for what the synchronous entry points upload and
+    // fetch: index tables, statuses, a container's bytes.  Grown on demand up
+    // to hh::kHostStageMax, kept until the context is destroyed; free
+    // whenever no entry point of the context runs (each waits for its own
+    // copies).
+    uint8_t *h_stage = nullptr;
+    size_t stage_bytes = 0;
     // Whole-matrix DCT bases as f16 hi / lo planes (dct_gemm.hip), two
     // cached: kind 0 B_n, 1 B_n^T, 2 the even / odd split of B_n^T.
     struct Basis {
@@ -68,6 +76,12 @@ int32_t check_hctt_tensor(const hh_hctt_tensor &T, size_t *ntiles);
 // (capi.hip).
 int32_t from_hip(hipError_t e);
 int32_t ensure_scratch(hh_context *ctx, size_t bytes);
+// ctx->h_stage grown to at least `bytes` with its first `keep` bytes kept
+// (capi.hip); nullptr above kHostStageMax or when the memory is not to be
+// had, in which case the caller takes ordinary memory.  The context's device
+// is current.
+constexpr size_t kHostStageMax = 32u << 20;
+uint8_t *host_stage(hh_context *ctx, size_t bytes, size_t keep);
 // Device address of the no-allocation entry point's array on `device`
 // (which must be current), looked up once per device (capi_noalloc.hip).
 hipError_t noalloc_scratch(int device, uint8_t **out);
@@ -358,8 +372,6 @@ int32_t dct2d_lines(hh_context *ctx, bool inverse, const float *d_in, uint32_t h
 int32_t hct3_decode_lines(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrags, bool coef_f32, uint32_t h,
                           uint32_t w, int32_t dtype, void *d_out, hipStream_t s);
 void release_line_tables(hh_context *ctx);
-// zstd::decode_all on the host (host_zstd.cpp): false on a malformed stream.
-bool zstd_decode_all(const uint8_t *in, size_t len, std::vector<uint8_t> &out);
 
 // Decodes n tensors (validated by the caller) in ceil(n/8) launches.
 hipError_t launch_hctt_decode(const hh_hctt_tensor *tensors, uint32_t n, int dtype,

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../include/haagenti_hip.h"
+#include "host_bytes.hpp"
 
 namespace {
 
@@ -426,7 +427,7 @@ size_t seq_table(FseTable &T, bool &have, int mode, const uint8_t *src, size_t l
     }
 }
 
-void decode_block(FrameState &F, const uint8_t *src, size_t len, std::vector<uint8_t> &out) {
+void decode_block(FrameState &F, const uint8_t *src, size_t len, hh::HostBytes &out) {
     if (len < 1) throw Fail{};
     // ---- literals section
     const uint8_t b0 = src[0];
@@ -526,7 +527,7 @@ void decode_block(FrameState &F, const uint8_t *src, size_t len, std::vector<uin
     }
     size_t lp = 0;
     if (nseq == 0) {
-        out.insert(out.end(), lit.begin(), lit.end());
+        out.append(lit.data(), lit.size());
         if (p != len) throw Fail{};
         return;
     }
@@ -572,7 +573,7 @@ void decode_block(FrameState &F, const uint8_t *src, size_t len, std::vector<uin
         }
         // execute: literals, then the match
         if (lp + ll > lit.size()) throw Fail{};
-        out.insert(out.end(), lit.begin() + lp, lit.begin() + lp + ll);
+        out.append(lit.data() + lp, ll);
         lp += ll;
         const size_t produced = out.size() - F.frame_start;
         if (off > produced || off > F.window) throw Fail{};
@@ -593,10 +594,10 @@ void decode_block(FrameState &F, const uint8_t *src, size_t len, std::vector<uin
         if (br.overflow()) throw Fail{};
     }
     if (br.pos != 0) throw Fail{};
-    out.insert(out.end(), lit.begin() + lp, lit.end());
+    out.append(lit.data() + lp, lit.size() - lp);
 }
 
-void decode_frames(const uint8_t *in, size_t len, std::vector<uint8_t> &out) {
+void decode_frames(const uint8_t *in, size_t len, hh::HostBytes &out) {
     size_t p = 0;
     if (len == 0) throw Fail{};
     while (p < len) {
@@ -656,12 +657,12 @@ void decode_frames(const uint8_t *in, size_t len, std::vector<uint8_t> &out) {
             if (btype == 3) throw Fail{};
             if (btype == 1) {
                 if (p >= len) throw Fail{};
-                out.insert(out.end(), bsize, in[p]);
+                out.append(bsize, in[p]);
                 p += 1;
             } else {
                 if (len - p < bsize) throw Fail{};
                 if (btype == 0) {
-                    out.insert(out.end(), in + p, in + p + bsize);
+                    out.append(in + p, bsize);
                 } else {
                     if (bsize > block_max && block_max) throw Fail{};
                     const size_t before = out.size();
@@ -688,7 +689,7 @@ void decode_frames(const uint8_t *in, size_t len, std::vector<uint8_t> &out) {
 namespace hh {
 // zstd::decode_all: every frame of the stream, concatenated.  Returns false
 // on a malformed stream.
-bool zstd_decode_all(const uint8_t *in, size_t len, std::vector<uint8_t> &out) {
+bool zstd_decode_all(const uint8_t *in, size_t len, HostBytes &out) {
     out.clear();
     try {
         decode_frames(in, len, out);
@@ -704,14 +705,14 @@ extern "C" {
 
 int32_t hh_zstd_decompress(const uint8_t *in, size_t in_len, uint8_t *out, size_t out_cap, size_t *written) {
     if ((!in && in_len) || !written) return HH_ERR_INVALID_ARGUMENT;
-    std::vector<uint8_t> v;
+    hh::HostBytes v;
     if (!hh::zstd_decode_all(in, in_len, v)) {
         *written = 0;
         return HH_ERR_CORRUPTED_DATA;
     }
     *written = v.size();
     if (v.size() > out_cap) return HH_ERR_BUFFER_TOO_SMALL;
-    if (!v.empty()) std::memcpy(out, v.data(), v.size());
+    if (v.size()) std::memcpy(out, v.data(), v.size());
     return HH_OK;
 }
 

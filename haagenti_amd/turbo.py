@@ -16,6 +16,8 @@ import json
 import mmap
 import struct
 
+import numpy as np
+
 from . import (BlockStatus, CHECKSUM_MISMATCH, CORRUPTED_DATA, F32, HaagentiError, OK, _addr, _lib, _sz, _u32,
                _torch_dtype, hct3_container, xxh3_64, xxh64, zstd_decompress)
 import ctypes as C
@@ -137,10 +139,13 @@ class TurboReader:
         w, h = dims(shape)
         if d_out is None:
             d_out = torch.empty(max(w * h, 1), dtype=_torch_dtype(dtype), device="cuda")
-        b = bytes(self.tensor_bytes(name))
+        b = self.tensor_bytes(name)
+        n = len(b)
+        b = np.frombuffer(b if n else bytes(1), np.uint8)  # in place: the map's or the file's own bytes
         ww, hh, st = _u32(0), _u32(0), BlockStatus()
-        rc = _lib.hh_turbo_tensor_decode(ctx.handle, b, len(b), 1 if verify else 0, int(dtype), _addr(d_out),
-                                         d_out.numel(), C.byref(ww), C.byref(hh), C.byref(st), stream)
+        rc = _lib.hh_turbo_tensor_decode(ctx.handle, b.ctypes.data, n, 1 if verify else 0, int(dtype),
+                                         _addr(d_out), d_out.numel(), C.byref(ww), C.byref(hh), C.byref(st), stream)
+        del b  # a view of the map, which close() releases
         if rc != OK:
             raise HaagentiError(rc, f"turbo tensor {name}", st)
         if (ww.value, hh.value) != (w, h):
