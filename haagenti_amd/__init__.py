@@ -450,8 +450,8 @@ class HipContext:
 
     def hctt_decode_lz4_batch(self, d_in, in_total, d_in_off, d_in_len, d_scratch, d_out_off, d_out_cap,
                               nblocks, d_status, tensors, dtype=F32, stream=None):
-        """LZ4 blocks -> scratch -> tiles of several tensors, two launches on
-        one stream (hh_hctt_decode_lz4_batch); tensors as for
+        """LZ4 blocks -> scratch -> tiles of several tensors, ordered on the
+        stream (hh_hctt_decode_lz4_batch); tensors as for
         hctt_decode_batch, their d_tiles inside d_scratch."""
         arr = (HcttTensor * len(tensors))()
         for i, t in enumerate(tensors):

@@ -2,6 +2,7 @@
 // Declarations and the reference interface each one replaces are in
 // include/haagenti_hip.h.
 #include <cmath>
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -197,6 +198,9 @@ void hh_context_destroy(hh_context *ctx) {
     if (ctx->d_basis) (void)hipFree(ctx->d_basis);
     if (ctx->d_scratch) (void)hipFree(ctx->d_scratch);
     if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
+    if (ctx->side) (void)hipStreamDestroy(ctx->side);
+    if (ctx->fork) (void)hipEventDestroy(ctx->fork);
+    if (ctx->join) (void)hipEventDestroy(ctx->join);
     hh::release_dct_resources(ctx);
     hh::release_fft_resources(ctx);
     hh::release_line_tables(ctx);
@@ -358,14 +362,165 @@ int32_t hh_hctt_decode_batch(hh_context *ctx, const hh_hctt_tensor *tensors, uin
                                            pick_stream(ctx, stream)));
 }
 
+namespace {
+
+// Dense tiles from which a layer is split (SparseSplit): the two streams'
+// events cost ~8 us a call, and what is hidden grows with the tiles.  Layers
+// of retention 0.10-0.50 at hidden 1024 (2,112 dense tiles) took 200 split
+// against 195 us, at 2048 (8,448) 210 against 223, at 4096 (37,888) 247
+// against 326.
+constexpr uint64_t kSplitTiles = 6144;
+
+// Whether a call on `s` may use the context's second stream, created with the
+// first such call: not while `s` is being captured, so that the second stream
+// never belongs to a capture that a later call would disturb.
+bool have_side(hh_context *ctx, hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (cap != hipStreamCaptureStatusNone) return false;
+    if (ctx->side) return true;
+    hipStream_t side = nullptr;
+    hipError_t e = ctx->fork ? hipSuccess : hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming);
+    if (e == hipSuccess && !ctx->join) e = hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    ctx->side = side;
+    return true;
+}
+
+// A layer with tensors on both sides of k = 1024 in two halves: the sparse
+// tensors' blocks with the sequence-batched decoder on the caller's stream,
+// beside the other blocks with the ring decoder and their tiles on the
+// context's second stream; then the sparse tensors' tiles.  A sparse block is
+// a chain of ~1,400 sequences on one wave (190 us at retention 0.10, three
+// waves to a CU), which one LZ4 launch makes every tile wait for: a
+// Llama-3-8B layer of retention 0.10-0.50 took 326 us that way (LZ4 190,
+// tiles 130), 247 split (chains 217 beside 42 + 146, then 43 for the sparse
+// tiles).  The dense tiles of 16-bit outputs run in four turns of
+// workgroups: the chains' waves take the place of some of them, which would
+// otherwise start when the others end (238 against 213 us at retention
+// 0.20-0.30); f32's leave room for both (296 us, in three turns 305).
+struct SparseSplit {
+    std::vector<hh_hctt_tensor> dense, sparse;
+    struct Span {
+        uint64_t lo, hi;
+    };
+    std::vector<Span> runs;  // the sparse tensors' tile bytes, joined where they touch
+    uint32_t first = 0;
+
+    static bool meet(const Span &a, const Span &b) { return a.lo < b.hi && b.lo < a.hi; }
+
+    // Whether the call takes this route: the decoder not chosen by the
+    // caller, valid tensors of both kinds, enough dense tiles to hide a
+    // chain behind, and nothing the halves write (tile bytes, weights,
+    // statuses) shared with what the other one reads or writes.
+    bool plan(const hh_context *ctx, const uint8_t *d_in, size_t in_total, const uint64_t *d_in_off,
+              const uint32_t *d_in_len, const uint8_t *d_scratch, const uint64_t *d_out_off,
+              const uint32_t *d_out_cap, uint32_t nblocks, const hh_block_status *d_status,
+              const hh_hctt_tensor *tensors, uint32_t n, int32_t dtype) {
+        if (ctx->lz4_decoder != HH_LZ4_AUTO || nblocks == 0 || n < 2 || n > 64) return false;
+        if (!d_in || !d_in_off || !d_in_len || !d_scratch || !d_out_off || !d_out_cap || !d_status) return false;
+        if (dtype != HH_F32 && dtype != HH_F16 && dtype != HH_BF16) return false;
+        auto span = [](const void *p, uint64_t bytes) {
+            return Span{(uint64_t)(uintptr_t)p, (uint64_t)(uintptr_t)p + bytes};
+        };
+        const uint64_t esz = dtype == HH_F32 ? 4 : 2;
+        // what the LZ4 halves read and write beside the tile bytes
+        std::vector<Span> fixed = {span(d_in, in_total), span(d_in_off, 8ull * nblocks), span(d_in_len, 4ull * nblocks),
+                                   span(d_out_off, 8ull * nblocks), span(d_out_cap, 4ull * nblocks),
+                                   span(d_status, sizeof(hh_block_status) * (uint64_t)nblocks)};
+        std::vector<Span> dtiles, stiles, douts, souts;
+        uint64_t ndense = 0, nsparse = 0;
+        for (uint32_t i = 0; i < n; i++) {
+            size_t nt = 0;
+            if (hh::check_hctt_tensor(tensors[i], &nt) != HH_OK) return false;
+            if (nt == 0) continue;
+            const bool sp = tensors[i].k < 1024u;
+            (sp ? sparse : dense).push_back(tensors[i]);
+            (sp ? nsparse : ndense) += nt;
+            (sp ? stiles : dtiles).push_back(span(tensors[i].d_tiles, nt * (uint64_t)hh_hctt_tile_bytes(tensors[i].k)));
+            (sp ? souts : douts).push_back(span(tensors[i].d_out, 4096ull * nt * esz));
+            if (tensors[i].d_tile_status) (sp ? souts : douts).push_back(span(tensors[i].d_tile_status, 4ull * nt));
+        }
+        if (nsparse == 0 || ndense < kSplitTiles || ndense + nsparse > 0xffffffffu) return false;
+        fixed.insert(fixed.end(), stiles.begin(), stiles.end());
+        for (const Span &t : dtiles)
+            for (const Span &f : fixed)
+                if (meet(t, f)) return false;
+        for (const Span &o : douts) {
+            for (const Span &f : fixed)
+                if (meet(o, f)) return false;
+            for (const Span &f : souts)
+                if (meet(o, f)) return false;
+        }
+        std::sort(stiles.begin(), stiles.end(), [](const Span &a, const Span &b) { return a.lo < b.lo; });
+        for (const Span &t : stiles) {
+            if (!runs.empty() && t.lo <= runs.back().hi)
+                runs.back().hi = t.hi > runs.back().hi ? t.hi : runs.back().hi;
+            else
+                runs.push_back(t);
+        }
+        first = hh::lz4_first_block(tensors, n, nblocks);
+        return runs.size() <= hh::kLz4Ranges;
+    }
+
+    hipError_t launch(hh_context *ctx, hh::Lz4Batch B, int32_t dtype, hipStream_t s) const {
+        B.nrange = (uint32_t)runs.size();
+        for (uint32_t i = 0; i < B.nrange; i++) {
+            B.lo[i] = runs[i].lo;
+            B.hi[i] = runs[i].hi;
+        }
+        hipError_t e = hipEventRecord(ctx->fork, s);
+        if (e == hipSuccess) e = hipStreamWaitEvent(ctx->side, ctx->fork, 0);
+        if (e != hipSuccess) return e;
+        // the chains start first and go straight on to their tiles
+        B.part = hh::kPartIn;
+        B.first = first;
+        const hipError_t ea = hh::launch_lz4_batch(B, HH_LZ4_SEQ, s);
+        B.part = hh::kPartOut;
+        B.first = 0;
+        e = hh::launch_lz4_batch(B, HH_LZ4_RING4, ctx->side);
+        if (e == hipSuccess)
+            e = hh::launch_hctt_decode(dense.data(), (uint32_t)dense.size(), dtype, ctx->d_basis, ctx->num_cus,
+                                       ctx->side, dtype == HH_F32 ? 1u : 4u);
+        // joined in any case: the caller's stream is after all of the call's work
+        hipError_t ej = hipEventRecord(ctx->join, ctx->side);
+        if (ej == hipSuccess) ej = hipStreamWaitEvent(s, ctx->join, 0);
+        if (e == hipSuccess) e = ea;
+        if (e == hipSuccess) e = ej;
+        if (e != hipSuccess) return e;
+        return hh::launch_hctt_decode(sparse.data(), (uint32_t)sparse.size(), dtype, ctx->d_basis, ctx->num_cus, s);
+    }
+};
+
+}  // namespace
+
 int32_t hh_hctt_decode_lz4_batch(hh_context *ctx, const uint8_t *d_in, size_t in_total, const uint64_t *d_in_off,
                                  const uint32_t *d_in_len, uint8_t *d_scratch, const uint64_t *d_out_off,
                                  const uint32_t *d_out_cap, uint32_t nblocks, hh_block_status *d_status,
                                  const hh_hctt_tensor *tensors, uint32_t ntensors, int32_t out_dtype,
                                  void *stream) {
-    // both launches on the caller's stream: the tile decode reads the
-    // scratch after every block has been written
     if (!ctx || (!tensors && ntensors)) return HH_ERR_INVALID_ARGUMENT;
+    SparseSplit sp;
+    if (sp.plan(ctx, d_in, in_total, d_in_off, d_in_len, d_scratch, d_out_off, d_out_cap, nblocks, d_status, tensors,
+                ntensors, out_dtype)) {
+        hh::DeviceGuard guard(ctx->device);
+        hipStream_t s = pick_stream(ctx, stream);
+        std::lock_guard<std::mutex> lock(ctx->side_lock);
+        if (guard.status() == hipSuccess && have_side(ctx, s)) {
+            const hh::Lz4Batch B = {d_in,      in_total,  d_in_off, d_in_len, d_scratch, ~0ull,
+                                    d_out_off, d_out_cap, nblocks,  d_status, 1u};
+            return from_hip(sp.launch(ctx, B, out_dtype, s));
+        }
+    }
+    // otherwise both launches on the caller's stream: the tile decode reads
+    // the scratch after every block has been written
     int32_t rc = lz4_batch_with(ctx, hh::lz4_decoder_for_tiles(ctx, tensors, ntensors), d_in, in_total, d_in_off,
                                 d_in_len, d_scratch, d_out_off, d_out_cap, nblocks, d_status, stream, true,
                                 hh::lz4_first_block(tensors, ntensors, nblocks));

@@ -1168,7 +1168,7 @@ __global__ __launch_bounds__(64 * kFusedMaxWaves) void hctt_lz4_fused_kernel(Til
 }  // namespace
 
 hipError_t launch_hctt_decode(const hh_hctt_tensor *tensors, uint32_t n, int dtype,
-                              const void *d_basis, int num_cus, hipStream_t s) {
+                              const void *d_basis, int num_cus, hipStream_t s, uint32_t turns) {
     // each launch takes the next (up to) kMaxTensors non-empty tensors
     for (uint32_t i = 0; i < n;) {
         TileBatch B;
@@ -1216,7 +1216,7 @@ hipError_t launch_hctt_decode(const hh_hctt_tensor *tensors, uint32_t n, int dty
         uint32_t per_cu = (uint32_t)kWavesPerSimd(dtype, np);
         if (per_cu > (160u * 1024u) / lds) per_cu = (160u * 1024u) / lds;
         if (per_cu == 0) per_cu = 1;
-        uint32_t grid = (uint32_t)(num_cus > 0 ? num_cus : 256) * per_cu;
+        uint32_t grid = (uint32_t)(num_cus > 0 ? num_cus : 256) * per_cu * turns;
         const uint32_t need = (total + kWaves - 1) / kWaves;
         if (grid > need) grid = need;
         const u32x4 *basis = reinterpret_cast<const u32x4 *>(d_basis);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <vector>
 
 #include "../../include/haagenti_hip.h"
@@ -64,6 +65,14 @@ struct hh_context {
     FftTables line_tab[8];  // dct_lines.hip
     void *d_fft = nullptr;
     size_t fft_bytes = 0;
+    // Second stream of hh_hctt_decode_lz4_batch with the events that order
+    // it after the caller's stream and the caller's stream after it (created
+    // with the first call that uses it; every use is joined again before the
+    // call returns).  The lock keeps one thread's event records and waits
+    // together.
+    std::mutex side_lock;
+    hipStream_t side = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr;
 };
 
 namespace hh {
@@ -173,6 +182,9 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float f) {
 hipError_t launch_dequant_int4(const uint8_t *d_q, size_t n, size_t nscale_groups,
                                int dtype, void *d_out, int num_cus, hipStream_t s);
 
+// which of a batch's blocks a launch decodes (Lz4Batch::part)
+enum : uint32_t { kPartAll = 0, kPartIn = 1, kPartOut = 2 };
+constexpr uint32_t kLz4Ranges = 8;
 // One batched LZ4 decode: block i reads in[in_off[i], +in_len[i]) (ranges
 // outside [0, in_total) are reported as HH_ERR_INVALID_ARGUMENT) and writes
 // at most out_cap[i] bytes at out + out_off[i]; a block whose output range
@@ -195,7 +207,19 @@ struct Lz4Batch {
     // the block the sequence-batched launch starts with (the others follow,
     // wrapping around), see lz4_first_block
     uint32_t first = 0;
+    // kPartIn: only the blocks whose output lies inside one of the nrange
+    // address ranges [lo, hi); kPartOut: only the others (ring and
+    // sequence-batched decoders)
+    uint32_t part = kPartAll, nrange = 0;
+    uint64_t lo[kLz4Ranges] = {}, hi[kLz4Ranges] = {};
 };
+__device__ __forceinline__ bool lz4_in_part(const Lz4Batch &B, uint64_t oofs, uint32_t ocap) {
+    if (B.part == kPartAll) return true;
+    const uint64_t a = (uint64_t)(uintptr_t)B.out + oofs;
+    bool in = false;
+    for (uint32_t i = 0; i < B.nrange; i++) in = in || (a >= B.lo[i] && a <= B.hi[i] && ocap <= B.hi[i] - a);
+    return in == (B.part == kPartIn);
+}
 
 // Batched LZ4 with the decoder `decoder` (hh_lz4_decoder; HH_LZ4_AUTO is
 // resolved by the caller): the sequence-batched decoder (lz4_seq.hip), the
@@ -373,9 +397,10 @@ int32_t hct3_decode_lines(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrag
                           uint32_t w, int32_t dtype, void *d_out, hipStream_t s);
 void release_line_tables(hh_context *ctx);
 
-// Decodes n tensors (validated by the caller) in ceil(n/8) launches.
+// Decodes n tensors (validated by the caller) in ceil(n/8) launches, each of
+// `turns` times the workgroups that fit the device at once.
 hipError_t launch_hctt_decode(const hh_hctt_tensor *tensors, uint32_t n, int dtype,
-                              const void *d_basis, int num_cus, hipStream_t s);
+                              const void *d_basis, int num_cus, hipStream_t s, uint32_t turns = 1);
 // LZ4 blocks of whole tiles decoded and their tiles decoded from LDS in one
 // launch per 8 tensors (hctt_decode.hip; validated by the caller: tensor i's
 // blocks are the next ceil(ntiles_i / tpb[i]) of d_in_off / d_in_len, each

@@ -20,6 +20,7 @@ __global__ __launch_bounds__(64) void lz4_ring_kernel(Lz4Batch B) {
     const uint32_t ilen = B.in_len[b];
     const uint64_t oofs = B.out_off[b];
     const uint32_t ocap = B.out_cap[b];
+    if (!lz4_in_part(B, oofs, ocap)) return;
     const bool out_ok = oofs <= B.out_total && (uint64_t)ocap <= B.out_total - oofs;
     uint8_t *out = B.out + oofs;
     D d;

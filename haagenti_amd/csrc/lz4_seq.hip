@@ -21,6 +21,11 @@ __global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B) {
     const uint32_t ilen = B.in_len[b];
     const uint64_t oofs = B.out_off[b];
     const uint32_t ocap = B.out_cap[b];
+    if (!lz4_in_part(B, oofs, ocap)) return;
+    // beside other kernels (a split layer) the chain issues before them:
+    // 217 against 265 us for a Llama-3-8B layer's tensors of retention 0.10
+    // and 0.20 (190 with the device to itself)
+    if (B.part == kPartIn) __builtin_amdgcn_s_setprio(3);
     const bool out_ok = oofs <= B.out_total && (uint64_t)ocap <= B.out_total - oofs;
     uint8_t *out = B.out + oofs;
     D d;

@@ -250,8 +250,12 @@ int32_t hh_hctt_decode_batch(hh_context *ctx, const hh_hctt_tensor *tensors, uin
 /* LZ4-compressed HCT-T tiles of several tensors in one call: every block of
  * d_in is decoded into d_scratch (hh_lz4_decompress_batch semantics, one
  * status record per block in d_status), then the tensors, whose d_tiles point
- * into d_scratch, are decoded (hh_hctt_decode_batch semantics); both launches
- * are queued on `stream` with no host synchronization.  This is what
+ * into d_scratch, are decoded (hh_hctt_decode_batch semantics); all of it is
+ * ordered on `stream` with no host synchronization (a large layer with
+ * tensors on both sides of k = 1024 decodes the two kinds beside each other,
+ * one of them on a stream of the context's that starts after the work queued
+ * on `stream` and that `stream` waits for; not while `stream` is captured).
+ * This is what
  * HctReader::decompress_all (haagenti-hct/src/tensor.rs:417-515) followed by
  * GpuDecompressor::decompress_batch_to_gpu (haagenti-cuda/src/decompress.rs:
  * 282-293) does for one layer's tensors.  A block that fails leaves its
