@@ -686,7 +686,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd(DT, NP)) void hctt_decode_k
 //
 // The input stage holds 8 KiB of a block's compressed bytes (a 16 KiB block
 // is staged in two or three batches of loads): it fits a wave's tile area,
-// which leaves the rest of the LDS to three block buffers.
+// which leaves the rest of the LDS to three block buffers (five with the batched decoder, launch_hctt_lz4_fused).
 constexpr uint32_t kFusedStageData = 8 * 1024;
 using FusedRing = ring::RingDec<16384, kFusedStageData, true>;
 using FusedSeq = seq::SeqDec<16384, kFusedStageData - 1024, true>;
@@ -699,7 +699,8 @@ constexpr uint32_t kFusedStageSeq = FusedSeq::kStageLds + FusedSeq::kTabLds + Fu
 constexpr uint32_t kFusedStage = kFusedStageRing > kFusedStageSeq ? kFusedStageRing : kFusedStageSeq;
 static_assert(FusedRing::kSFront == FusedSeq::kSFront, "both decoders' stages start at the same offset");
 constexpr int kFusedMaxWaves = 12;     // 3 per SIMD: 168 registers, tile_body's budget
-constexpr uint32_t kFusedMaxBufs = 4;
+constexpr int kFusedSeqWaves = 8;      // with the batched decoder (launch_hctt_lz4_fused)
+constexpr uint32_t kFusedMaxBufs = 5;
 constexpr uint32_t kFusedLdsMax = 160u * 1024u;
 constexpr uint32_t kSpinLimit = 1u << 24;  // polls of about 64 cycles each
 constexpr uint32_t kFusedMaxRange = 512;  // slots per workgroup (the bitmaps' size)
@@ -722,8 +723,8 @@ struct FusedBlocks {
     uint32_t spin_limit;                  // polls before a wait gives up
 };
 
-// Workgroup LDS layout after the shared part: [block descriptor][state[8]
-// (8 bytes each), done[8], abort, next_block, next_tile, finished, left,
+// Workgroup LDS layout after the shared part: [block descriptor][state[5]
+// (8 bytes each), done[5], abort, next_block, next_tile, finished, left,
 // the complete and failed bitmaps][wave areas][block buffers].
 constexpr uint32_t kFusedFOff = kSharedBytes;
 constexpr uint32_t kFusedFlagsOff = kFusedFOff + ((sizeof(FusedBlocks) + 15u) & ~15u);
@@ -742,6 +743,8 @@ constexpr uint32_t kFusedWaveOff = kFusedFlagsOff + ((4 * kFusedFlagWords + 15u)
 // waves with a whole-tile park each and three block buffers
 static_assert(kFusedWaveOff + 12u * 64u * kParkPitch<HH_BF16> + 3u * kFusedBuf <= kFusedLdsMax,
               "twelve waves and three block buffers fit the LDS");
+static_assert(kFusedWaveOff + kFusedSeqWaves * 64u * kParkPitch<HH_BF16> + 5u * kFusedBuf <= kFusedLdsMax,
+              "eight waves and five block buffers fit the LDS");
 
 typedef uint32_t __attribute__((address_space(3))) lds_word;
 typedef uint64_t __attribute__((address_space(3))) lds_dword;
@@ -1307,13 +1310,22 @@ hipError_t launch_hctt_lz4_fused(const hh_hctt_tensor *tensors, uint32_t n, cons
         const uint32_t obytes = 64 * (dtype == HH_F32 ? kParkPitch<HH_F32> : kParkPitch<HH_BF16>);
         B.vo_bytes = ((vbytes > obytes ? vbytes : obytes) + 15u) & ~15u;
         B.wave_lds = B.vo_bytes > kFusedStage ? B.vo_bytes : (kFusedStage + 15u) & ~15u;
-        // one workgroup per CU: kFusedMaxWaves waves (fewer when their areas
-        // leave room for fewer than 3 block buffers)
-        uint32_t nw = kFusedMaxWaves, nbuf = 0;
+        // One workgroup per CU: kFusedMaxWaves waves (fewer when their areas
+        // leave room for fewer than 3 block buffers).  With the batched
+        // decoder a block is a long chain on one wave, and what bounds the
+        // launch is how many are decoded at once: 8 waves, which leave room
+        // for 5 buffers (f32 parks: 5 waves and 4).  A Llama-3-8B layer to
+        // bf16, 12 waves and 3 buffers / 10 and 4 / 8 and 5 / 6 and 6:
+        // retention 0.10 754 / 626 / 454 / 491 us, 0.20 418 / 335 / 299 /
+        // 326, 0.10-0.50 402 / 384 / 367 / 386; to f32 at 0.10, 6 and 3 / 5
+        // and 4 / 4 and 5: 718 / 602 / 622.  The ring decoder's short chains
+        // keep 12 (retention 0.30: 173 us, 9 and 4 179, 8 and 5 184).
+        uint32_t nw = seq_decoder ? kFusedSeqWaves : kFusedMaxWaves, nbuf = 0;
+        const uint32_t want = seq_decoder && dtype == HH_F32 ? 4u : 3u;
         for (;;) {
             const uint32_t used = kFusedWaveOff + nw * B.wave_lds;
             nbuf = used < kFusedLdsMax ? (kFusedLdsMax - used) / kFusedBuf : 0u;
-            if (nbuf >= 3 || nw == 1) break;
+            if (nbuf >= want || nw == 1) break;
             nw--;
         }
         if (nbuf < 2) return hipErrorInvalidValue;  // not reached: tiles are at most 3 KiB (k <= 4096)

@@ -18,10 +18,10 @@ DENSE, DENSE2, SPARSE, SPARSE2 = (4096, 6144, 0.30), (512, 4096, 0.45), (1024, 2
 DTYPES = {"f32": 4, "f16": 2, "bf16": 2}
 
 
-def layer(specs, seed, cut=None, gap=0):
+def layer(specs, seed, cut=None, gap=0, most=1 << 30):
     """The tensors' tile bytes one after another (`gap` bytes between them),
-    in blocks of whole tiles or, with `cut`, of that many bytes across the
-    tensors.  A tensor repeats 64 encoded tiles."""
+    in blocks of whole tiles (`most` of them at most) or, with `cut`, of that
+    many bytes across the tensors.  A tensor repeats 64 encoded tiles."""
     import haagenti_amd as H
     rng = np.random.default_rng(seed)
     comp = H.Lz4Compressor()
@@ -39,7 +39,8 @@ def layer(specs, seed, cut=None, gap=0):
     else:
         starts = []
         for t in tensors:
-            per = 16352 // H.hctt_tile_bytes(t["k"]) * H.hctt_tile_bytes(t["k"])
+            t["per"] = min(most, 16352 // H.hctt_tile_bytes(t["k"]))
+            per = t["per"] * H.hctt_tile_bytes(t["k"])
             starts += [(a, min(a + per, t["soff"] + t["n"])) for a in range(t["soff"], t["soff"] + t["n"], per)]
     seen, blobs = {}, []
     for a, b in starts:
