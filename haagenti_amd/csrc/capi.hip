@@ -198,7 +198,6 @@ void hh_context_destroy(hh_context *ctx) {
     if (ctx->d_basis) (void)hipFree(ctx->d_basis);
     if (ctx->d_scratch) (void)hipFree(ctx->d_scratch);
     if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
-    if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->fork) (void)hipEventDestroy(ctx->fork);
     if (ctx->join) (void)hipEventDestroy(ctx->join);
     hh::release_dct_resources(ctx);
@@ -367,41 +366,39 @@ namespace {
 // Dense tiles from which a layer is split (SparseSplit): the two streams'
 // events cost ~8 us a call, and what is hidden grows with the tiles.  Layers
 // of retention 0.10-0.50 at hidden 1024 (2,112 dense tiles) took 200 split
-// against 195 us, at 2048 (8,448) 210 against 223, at 4096 (37,888) 247
+// against 195 us, at 2048 (8,448) 210 against 223, at 4096 (37,888) 244
 // against 326.
 constexpr uint64_t kSplitTiles = 6144;
 
-// Whether a call on `s` may use the context's second stream, created with the
-// first such call: not while `s` is being captured, so that the second stream
-// never belongs to a capture that a later call would disturb.
-bool have_side(hh_context *ctx, hipStream_t s) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
+// Whether a call on `s` may use the context's stream beside it: not while
+// either is being captured, so that the context's stream never belongs to a
+// capture that a later call would disturb.  (A stream of its own would be one
+// more on the device's four hardware queues, where a pipeline's copies then
+// waited behind its decodes.)
+bool may_split(hh_context *ctx, hipStream_t s) {
+    if (s == ctx->stream) return false;
+    for (hipStream_t x : {s, ctx->stream}) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(x, &cap) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (cap != hipStreamCaptureStatusNone) return false;
     }
-    if (cap != hipStreamCaptureStatusNone) return false;
-    if (ctx->side) return true;
-    hipStream_t side = nullptr;
     hipError_t e = ctx->fork ? hipSuccess : hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming);
     if (e == hipSuccess && !ctx->join) e = hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    ctx->side = side;
-    return true;
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
 }
 
 // A layer with tensors on both sides of k = 1024 in two halves: the sparse
 // tensors' blocks with the sequence-batched decoder on the caller's stream,
 // beside the other blocks with the ring decoder and their tiles on the
-// context's second stream; then the sparse tensors' tiles.  A sparse block is
+// context's own stream; then the sparse tensors' tiles.  A sparse block is
 // a chain of ~1,400 sequences on one wave (190 us at retention 0.10, three
 // waves to a CU), which one LZ4 launch makes every tile wait for: a
 // Llama-3-8B layer of retention 0.10-0.50 took 326 us that way (LZ4 190,
-// tiles 130), 247 split (chains 217 beside 42 + 146, then 43 for the sparse
+// tiles 130), 244 split (chains 217 beside 42 + 146, then 43 for the sparse
 // tiles).  The dense tiles of 16-bit outputs run in four turns of
 // workgroups: the chains' waves take the place of some of them, which would
 // otherwise start when the others end (238 against 213 us at retention
@@ -477,7 +474,7 @@ struct SparseSplit {
             B.hi[i] = runs[i].hi;
         }
         hipError_t e = hipEventRecord(ctx->fork, s);
-        if (e == hipSuccess) e = hipStreamWaitEvent(ctx->side, ctx->fork, 0);
+        if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, ctx->fork, 0);
         if (e != hipSuccess) return e;
         // the chains start first and go straight on to their tiles
         B.part = hh::kPartIn;
@@ -485,12 +482,12 @@ struct SparseSplit {
         const hipError_t ea = hh::launch_lz4_batch(B, HH_LZ4_SEQ, s);
         B.part = hh::kPartOut;
         B.first = 0;
-        e = hh::launch_lz4_batch(B, HH_LZ4_RING4, ctx->side);
+        e = hh::launch_lz4_batch(B, HH_LZ4_RING4, ctx->stream);
         if (e == hipSuccess)
             e = hh::launch_hctt_decode(dense.data(), (uint32_t)dense.size(), dtype, ctx->d_basis, ctx->num_cus,
-                                       ctx->side, dtype == HH_F32 ? 1u : 4u);
+                                       ctx->stream, dtype == HH_F32 ? 1u : 4u);
         // joined in any case: the caller's stream is after all of the call's work
-        hipError_t ej = hipEventRecord(ctx->join, ctx->side);
+        hipError_t ej = hipEventRecord(ctx->join, ctx->stream);
         if (ej == hipSuccess) ej = hipStreamWaitEvent(s, ctx->join, 0);
         if (e == hipSuccess) e = ea;
         if (e == hipSuccess) e = ej;
@@ -513,7 +510,7 @@ int32_t hh_hctt_decode_lz4_batch(hh_context *ctx, const uint8_t *d_in, size_t in
         hh::DeviceGuard guard(ctx->device);
         hipStream_t s = pick_stream(ctx, stream);
         std::lock_guard<std::mutex> lock(ctx->side_lock);
-        if (guard.status() == hipSuccess && have_side(ctx, s)) {
+        if (guard.status() == hipSuccess && may_split(ctx, s)) {
             const hh::Lz4Batch B = {d_in,      in_total,  d_in_off, d_in_len, d_scratch, ~0ull,
                                     d_out_off, d_out_cap, nblocks,  d_status, 1u};
             return from_hip(sp.launch(ctx, B, out_dtype, s));

@@ -65,13 +65,11 @@ struct hh_context {
     FftTables line_tab[8];  // dct_lines.hip
     void *d_fft = nullptr;
     size_t fft_bytes = 0;
-    // Second stream of hh_hctt_decode_lz4_batch with the events that order
-    // it after the caller's stream and the caller's stream after it (created
-    // with the first call that uses it; every use is joined again before the
-    // call returns).  The lock keeps one thread's event records and waits
-    // together.
+    // Events that order hh_hctt_decode_lz4_batch's work on `stream` after the
+    // caller's stream and the caller's stream after it (created with the
+    // first call that uses them; joined again before the call returns).  The
+    // lock keeps one thread's event records and waits together.
     std::mutex side_lock;
-    hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
 };
 

@@ -253,8 +253,8 @@ int32_t hh_hctt_decode_batch(hh_context *ctx, const hh_hctt_tensor *tensors, uin
  * into d_scratch, are decoded (hh_hctt_decode_batch semantics); all of it is
  * ordered on `stream` with no host synchronization (a large layer with
  * tensors on both sides of k = 1024 decodes the two kinds beside each other,
- * one of them on a stream of the context's that starts after the work queued
- * on `stream` and that `stream` waits for; not while `stream` is captured).
+ * one of them on hh_context_stream(), after the work queued on `stream`, which
+ * waits for it; not while either stream is captured).
  * This is what
  * HctReader::decompress_all (haagenti-hct/src/tensor.rs:417-515) followed by
  * GpuDecompressor::decompress_batch_to_gpu (haagenti-cuda/src/decompress.rs:

@@ -156,8 +156,7 @@ def test_outputs_over_the_compressed_input():
 
 def test_streams_threads_and_capture():
     T = G.torch()
-    import haagenti_amd as H
-    ctx = H.HipContext(0)
+    ctx = G.ctx()
     calls = [Call(layer([DENSE, SPARSE, SPARSE2], 5 + i), ctx=ctx) for i in range(3)]
     want = [general(c) for c in calls]
     for c in calls:
