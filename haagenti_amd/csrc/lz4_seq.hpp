@@ -337,8 +337,8 @@ struct SeqDec {
 
     // 16 bytes of output from virtual position sp on: from the ring when
     // their 20-byte window (from sp rounded down to 4) starts at or after
-    // rlo (written at most R bytes before the batch end), else from the
-    // written-out output.  The output's dwords are read at addresses clamped
+    // rlo (written less than R bytes before the batch end, see execute), else
+    // from the written-out output.  The output's dwords are read at addresses clamped
     // to the dwords holding the block's output bytes, so a window reaching
     // outside them reads no memory outside them (those bytes are never used:
     // they lie before a match's source).
@@ -737,7 +737,12 @@ struct SeqDec {
         const uint32_t len = ll + ml;
         const uint32_t vl = op_b + a0 + scan_add(len) - len;  // virtual start of the slot
         const uint32_t vm = vl + ll;
-        const int32_t rlo = (int32_t)(op + a0) - (int32_t)R;
+        // The ring's slots from the batch's end on hold the R bytes before it,
+        // but up to 15 of them may be the don't-care bytes of a long run's
+        // last chunk, in an earlier batch too when this one is shorter than
+        // that: the ring serves sources from rlo on, 32 bytes after its
+        // start, and what lies before is in the written-out output.
+        const int32_t rlo = (int32_t)(op + a0) - (int32_t)R + 32;
         if (op - op_b >= 256u * nsl) {
             // runs of 128 bytes or more on average: one run per pass
             for (uint32_t i = 0; i < nsl; i++) {
@@ -746,14 +751,12 @@ struct SeqDec {
                 const uint32_t m = rdl(ml, i);
                 if (m > 0) {
                     const uint32_t off = rdl(mo, i);
-                    // (ring slots up to 16 bytes past a run's end may hold its
-                    // don't-care bytes: the ring serves windows from rlo + 32)
                     if (off >= m)
-                        match_serial<0>(v + n, m, off, rlo + 32);
+                        match_serial<0>(v + n, m, off, rlo);
                     else if (off >= 16u)
-                        match_serial<1>(v + n, m, off, rlo + 32);
+                        match_serial<1>(v + n, m, off, rlo);
                     else
-                        match_serial<2>(v + n, m, off, rlo + 32);
+                        match_serial<2>(v + n, m, off, rlo);
                 }
             }
             return;

@@ -67,6 +67,50 @@ def test_short_sequences(case):
     check_against_oracle(broken, caps, out_pad=3)
 
 
+def after_long_run(rng, ring, first, mlen, off, tail=5):
+    """`first` literals and a match of `mlen` bytes from ring - 128 back
+    (copied as long runs, a batch that ends there), then a match of 4 from
+    `off` back and the last literals: a batch of 4 + `tail` bytes, whose
+    source lies where the long run's last chunk of 16 bytes ends."""
+    out = _seq(bytes(rng.integers(0, 256, first, dtype=np.uint8)), ring - 128, mlen)
+    out += _seq(b"", off, 4) + _seq(bytes(rng.integers(0, 256, tail, dtype=np.uint8)))
+    return out, first + mlen + 4 + tail
+
+
+@pytest.mark.parametrize("tail", [5, 7, 11, 13])
+def test_short_batch_after_a_long_run(decoder, tail):
+    # every alignment of the long run's end, sources around the ring's end
+    ring = 8192 if decoder == "seq8" else 4096
+    rng = np.random.default_rng(ring + tail)
+    items = [after_long_run(rng, ring, 2 * ring + 1900 + a, 61 + b, ring - o, tail)
+             for a in range(16) for b in (0, 1) for o in range(-2, 42)]
+    for out_align in (0, 9):
+        check_against_oracle([s for s, _ in items], [c for _, c in items], out_align=out_align, out_pad=3)
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_long_runs_between_short_sequences(decoder, seed):
+    # batches of long runs and of a few short sequences by turns
+    ring = 8192 if decoder == "seq8" else 4096
+    rng = np.random.default_rng(100 * seed + ring)
+    items = []
+    for _ in range(96):
+        out, size = bytearray(), 0
+        for _ in range(6):
+            n, m = int(rng.integers(300, 3000)), int(rng.integers(40, 80))
+            size += n
+            out += _seq(bytes(rng.integers(0, 256, n, dtype=np.uint8)), min(size, ring - 128 - int(rng.integers(3))), m)
+            size += m
+            for _ in range(int(rng.integers(1, 4))):
+                m, n = int(rng.integers(4, 7)), int(rng.integers(0, 3))
+                size += n
+                out += _seq(bytes(rng.integers(0, 256, n, dtype=np.uint8)), min(size, ring - int(rng.integers(-4, 64))), m)
+                size += m
+        out += _seq(bytes(rng.integers(0, 256, 5, dtype=np.uint8)))
+        items.append((bytes(out), size + 5))
+    check_against_oracle([s for s, _ in items], [c for _, c in items], out_align=seed * 5, out_pad=3)
+
+
 @pytest.mark.parametrize("rho", [0.05, 0.10, 0.15, 0.20])
 def test_sparse_tiles_on_both_routes(rho):
     import haagenti_amd as H
