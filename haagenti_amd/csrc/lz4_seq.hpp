@@ -127,7 +127,7 @@ __device__ __forceinline__ uint32_t umod(uint32_t x, uint32_t m) {
 }
 
 // Parse state between batches.
-enum : uint32_t { kToken = 0, kLit = 1, kOff = 2, kMatch = 3 };
+enum : uint32_t { kToken = 0, kLitExt = 1, kLit = 2, kOff = 3, kMatchExt = 4, kMatch = 5 };
 
 struct NoProgress {
     __device__ __forceinline__ void operator()(uint32_t) const {}
@@ -289,17 +289,15 @@ struct SeqDec {
     // Length extension from *pp (block.rs:277-289, 329-341) once 7 (or 6)
     // 0xFF bytes have been seen: adds 255 per 0xFF byte plus the first other
     // byte.  Returns 0 when done, 1 at the end of the block input (the
-    // reference reports UnexpectedEof), 2 when it needs bytes past the stage
-    // while the batch holds copies that read the stage (the caller ends the
-    // batch and parses the sequence again); with no such copies it restages.
-    __device__ __forceinline__ int ext_slow(uint32_t &pp, uint32_t end, uint64_t &len, bool pend) {
+    // reference reports UnexpectedEof), 2 where it goes on past the stage
+    // (the caller restages there or, where the batch holds copies that read
+    // the stage, ends the batch and parses the sequence again).
+    __device__ __forceinline__ int ext_slow(uint32_t &pp, uint32_t end, uint64_t &len) {
         uint32_t p = pp;
         for (;;) {
+            pp = p;
             if (p >= end) return 1;
-            if (!in_stage8(p)) {
-                if (pend) return 2;
-                restage(p);
-            }
+            if (!in_stage8(p)) return 2;
             const uint64_t x = read8(p);
             const uint64_t nz = ~x;
             if (nz == 0) {
@@ -479,6 +477,15 @@ struct SeqDec {
     __device__ __forceinline__ static uint32_t short_dist(uint32_t token, uint32_t next) {
         const uint32_t k = token >= 0xf0u ? 19u + next : (token >> 4) + 3u;
         return (token & 15u) == 15u || (token >= 0xf0u && next == 255u) ? 0u : k;
+    }
+    // Whether a walk starts at token t2 & 255 (t2 >> 8: the byte after it),
+    // `room` bytes before the walk's end: a short sequence of at most 48
+    // bytes.  Longer ones, one or two to a window of 256, are parsed faster
+    // one at a time (a Llama-3-8B layer of retention 0.24 209 -> 203 us).
+    __device__ __forceinline__ static bool walkable(uint32_t t2, uint32_t room) {
+        if ((t2 & 15u) == 15u) return false;
+        const uint32_t k = short_dist(t2 & 0xffu, (t2 >> 8) & 0xffu);
+        return k - 1u < 48u && k <= room;
     }
     // Finds the tokens of a run of such sequences from stage offset x0 on,
     // each next token at or before stage offset xe and no window past x_max:
@@ -870,6 +877,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
     uint32_t ip = 0;
     uint32_t ms = kToken;
     uint32_t lit_rem = 0, m_rem = 0, m_off = 0, tml = 0;
+    uint64_t acc = 0;  // kLitExt, kMatchExt: the length so far
     d.hv = 0;
     d.hb = 0;
     // the list of short sequences: next entry, entries, stage offset after them
@@ -892,8 +900,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
         // slots in lanes (slot i in lane i): literal stage offset and length,
         // match offset and length, token position (fast loop only)
         uint32_t ls = 0, ll = 0, mo = 0, ml = 0, tp = 0;
-        uint64_t walked = 0;  // slots of sequences from the list
-        uint32_t lslot = 64, lfirst = 0;  // the list's first slot of this batch and its entry
+        bool walked = false;  // the slot is a sequence from the list
         if (ms != kToken) nsl = 1;  // a run continued from the previous batch
         for (;;) {
             // ---- fast loop: header chain only
@@ -909,6 +916,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                 uint32_t fo = op;
                 uint32_t fl = lim < op_b + D::kOB ? lim : op_b + D::kOB;
                 bool full = false;
+                uint32_t lt = 0;  // how many of the last slots came from the list
                 // short sequences end inside the stage and the block
                 const uint32_t we = d.at_end || end - d.sb < S ? end - d.sb : S;
                 for (;;) {
@@ -917,9 +925,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                     if (nsl < 64u && fp <= hl && fo < fl) {
                         if (li == ln) {
                             if (!d.in_win8(fp)) d.read16(fp);
-                            const uint32_t t2 = (uint32_t)d.peek8(fp) & 0xffffu;
-                            const uint32_t k = D::short_dist(t2 & 0xffu, t2 >> 8);
-                            if (k != 0u && fp - d.sb + k <= we) {
+                            if (D::walkable((uint32_t)d.peek8(fp), we - (fp - d.sb))) {
                                 // (their output is at least their input: no
                                 // token past the batch's budget)
                                 lx = fp - d.sb;
@@ -939,11 +945,10 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                                 ml = (token & 15u) + 4u;
                                 mo = (uint32_t)d.stage[ls + ll] | ((uint32_t)d.stage[ls + ll + 1u] << 8);
                                 tp += d.sb;
+                                walked = true;
                             }
                             fo += rdl(scan_add(me ? ll + ml : 0u), 63);
-                            walked |= (~0ull >> (64u - n)) << w0;
-                            lslot = w0;
-                            lfirst = li;
+                            lt = n;
                             li += n;
                             nsl += n;
                             fp = d.sb + (li < ln ? rfl((uint32_t)d.list[li]) : lx);
@@ -957,12 +962,9 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                         const uint64_t t8 = d.peek8(fp);
                         const uint32_t token = (uint32_t)t8 & 0xffu;
                         uint32_t lit = token >> 4;
-                        if (any && fo < fl) {
-                            const uint32_t k = D::short_dist(token, (uint32_t)(t8 >> 8) & 0xffu);
-                            if (k != 0u && fp - d.sb + k <= we) {
-                                back = true;
-                                break;
-                            }
+                        if (any && fo < fl && D::walkable((uint32_t)t8, we - (fp - d.sb))) {
+                            back = true;
+                            break;
                         }
                         any = true;
                         uint32_t p = fp + 1;
@@ -1004,6 +1006,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                         mo = me ? off : mo;
                         ml = me ? mlen : ml;
                         nsl++;
+                        lt = 0;
                         fp = q;
                         fo = fm + mlen;
                         fl = fl2;
@@ -1022,7 +1025,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                     // near-match limit: prefix minimum over the fast slots
                     // (a walked sequence's match does not end the batch for a
                     // source that leaves the ring: it reads the output)
-                    uint32_t nl = (!LDS && lane >= f0 && live && mo <= R - 128u && !((walked >> lane) & 1ull))
+                    uint32_t nl = (!LDS && lane >= f0 && live && mo <= R - 128u && !walked)
                                       ? om - mo + (R - 64u)
                                       : 0xffffffffu;
                     nl = ~scan_max(~nl);
@@ -1039,12 +1042,12 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                     // a slot past the batch's budget or limit starts the next batch
                     if (f < nsl) full = (ballot(valid) >> f) & 1ull;
                     ip = f < nsl ? rdl(tp, f) : fp;
-                    // the list goes on with the first slot not kept
-                    if (f < nsl && li > 0) {
-                        if (lslot <= f && lslot < nsl)
-                            li = lfirst + (f - lslot);
-                        else
-                            li = ln = 0;
+                    // the list goes on with the first slot not kept, if
+                    // that came from it
+                    if (f < nsl) {
+                        const bool listed = nsl - f <= lt;
+                        li = listed ? li - (nsl - f) : 0u;
+                        ln = listed ? ln : 0u;
                     }
                     nsl = f;
                     const bool keep = lane < f;
@@ -1059,73 +1062,82 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                 if (full && bout > 0) break;
             }
             // ---- general step
-            if (ms == kToken) {
-                if (ip >= end) {
-                    done = true;
-                    break;
-                }
-                if (nsl == 64u) break;
-                if (!d.in_win8(ip) && !d.in_stage8(ip)) {
-                    restage = true;
-                    break;
-                }
+            if (ms <= kLitExt) {
                 // token and literal length (block.rs:270-289); the extension
                 // bytes usually lie in the 7 bytes after the token
-                const uint64_t t8 = d.get8(ip);
-                const uint32_t token = (uint32_t)t8 & 0xffu;
-                uint32_t lit = token >> 4;
-                uint32_t p = ip + 1;
-                if (lit == 15) {
-                    const uint64_t x = t8 >> 8;
-                    const uint64_t nz = ~x & 0x00ffffffffffffffull;
-                    if (nz != 0) {
-                        const uint32_t e = (uint32_t)__builtin_ctzll(nz) >> 3;
-                        if (p + e >= end) {
-                            code = HH_ERR_UNEXPECTED_EOF;
-                            pos = ilen;
-                            return;
-                        }
-                        lit += 255u * e + (uint32_t)((x >> (8 * e)) & 0xffu);
-                        p += e + 1;
-                    } else {
-                        uint64_t l64 = lit + 255ull * 7;
-                        p += 7;
-                        const int r = p >= end ? 1 : d.ext_slow(p, end, l64, bout != 0);
-                        if (r == 1) {
-                            code = HH_ERR_UNEXPECTED_EOF;
-                            pos = ilen;
-                            return;
-                        }
-                        if (r == 2) {  // parse this sequence again after the batch
-                            restage = true;
-                            break;
-                        }
-                        // a length beyond 32 bits exceeds the block input:
-                        // the input-length check below fails for it too
-                        if (l64 > 0xffffffffull) {
-                            code = HH_ERR_UNEXPECTED_EOF;
-                            pos = p;
-                            return;
-                        }
-                        lit = (uint32_t)l64;
+                uint32_t p = ip;
+                uint64_t lit;
+                bool ext = true;
+                if (ms == kToken) {
+                    if (ip >= end) {
+                        done = true;
+                        break;
                     }
+                    if (nsl == 64u) break;
+                    if (!d.in_win8(ip) && !d.in_stage8(ip)) {
+                        restage = true;
+                        break;
+                    }
+                    const uint64_t t8 = d.get8(ip);
+                    const uint32_t token = (uint32_t)t8 & 0xffu;
+                    tml = token & 15u;
+                    lit = token >> 4;
+                    p++;
+                    ext = false;
+                    if (lit == 15) {
+                        const uint64_t x = t8 >> 8;
+                        const uint32_t e = (uint32_t)__builtin_ctzll(~x | (1ull << 56)) >> 3;  // 7: none
+                        ext = e == 7u;
+                        if (!ext && p + e >= end) {
+                            code = HH_ERR_UNEXPECTED_EOF;
+                            pos = ilen;
+                            return;
+                        }
+                        lit += 255u * e + (ext ? 0u : (uint32_t)((x >> (8 * e)) & 0xffu));
+                        p += ext ? 7u : e + 1u;
+                    }
+                } else {
+                    lit = acc;
                 }
-                if (lit > 0) {
-                    if (end - p < lit) {
+                if (ext) {
+                    const int r = d.ext_slow(p, end, lit);
+                    if (r == 1) {
+                        code = HH_ERR_UNEXPECTED_EOF;
+                        pos = ilen;
+                        return;
+                    }
+                    if (r == 2) {
+                        if (bout == 0) {
+                            ip = p;
+                            acc = lit;
+                            ms = kLitExt;
+                        }
+                        restage = true;
+                        break;
+                    }
+                    // a length beyond 32 bits exceeds the block input:
+                    // the input-length check below fails for it too
+                    if (lit > 0xffffffffull) {
                         code = HH_ERR_UNEXPECTED_EOF;
                         pos = p;
                         return;
                     }
-                    if (lit > cap - op) {
+                }
+                lit_rem = (uint32_t)lit;
+                if (lit_rem > 0) {
+                    if (end - p < lit_rem) {
+                        code = HH_ERR_UNEXPECTED_EOF;
+                        pos = p;
+                        return;
+                    }
+                    if (lit_rem > cap - op) {
                         code = HH_ERR_BUFFER_TOO_SMALL;
-                        req = (uint64_t)op + lit;
+                        req = (uint64_t)op + lit_rem;
                         return;
                     }
                 }
-                nsl++;  // the sequence's slot (zero in every lane)
-                tml = token & 15u;
+                if (ms == kToken) nsl++;  // the sequence's slot (zero in every lane)
                 ip = p;
-                lit_rem = lit;
                 ms = kLit;
             }
             if (ms == kLit) {
@@ -1156,63 +1168,72 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                 }
                 ms = kOff;
             }
-            if (ms == kOff) {
+            if (ms == kOff || ms == kMatchExt) {
                 // offset and match length (block.rs:313-345)
-                if (end - ip < 2) {
-                    code = HH_ERR_UNEXPECTED_EOF;
-                    pos = ip;
-                    return;
-                }
-                if (!d.in_win8(ip) && !d.in_stage8(ip)) {
-                    restage = true;
-                    break;
-                }
-                const uint64_t o8 = d.get8(ip);
-                const uint32_t off = (uint32_t)o8 & 0xffffu;
-                uint32_t p = ip + 2;
-                if (off == 0) {
-                    code = HH_ERR_CORRUPTED_DATA;
-                    detail = HH_CORRUPT_ZERO_OFFSET;
-                    return;
-                }
-                if (off > op) {
-                    code = HH_ERR_CORRUPTED_DATA;
-                    detail = HH_CORRUPT_OFFSET_BEYOND;
-                    pos = op;
-                    return;
-                }
-                uint32_t mlen = tml + 4u;
-                if (tml == 15u) {
-                    const uint64_t x = o8 >> 16;
-                    const uint64_t nz = ~x & 0x0000ffffffffffffull;
-                    if (nz != 0) {
-                        const uint32_t e = (uint32_t)__builtin_ctzll(nz) >> 3;
-                        if (p + e >= end) {
+                uint32_t p = ip;
+                uint64_t mlen;
+                bool ext = true;
+                if (ms == kOff) {
+                    if (end - ip < 2) {
+                        code = HH_ERR_UNEXPECTED_EOF;
+                        pos = ip;
+                        return;
+                    }
+                    if (!d.in_win8(ip) && !d.in_stage8(ip)) {
+                        restage = true;
+                        break;
+                    }
+                    const uint64_t o8 = d.get8(ip);
+                    m_off = (uint32_t)o8 & 0xffffu;
+                    p += 2;
+                    if (m_off == 0) {
+                        code = HH_ERR_CORRUPTED_DATA;
+                        detail = HH_CORRUPT_ZERO_OFFSET;
+                        return;
+                    }
+                    if (m_off > op) {
+                        code = HH_ERR_CORRUPTED_DATA;
+                        detail = HH_CORRUPT_OFFSET_BEYOND;
+                        pos = op;
+                        return;
+                    }
+                    mlen = tml + 4u;
+                    ext = false;
+                    if (tml == 15u) {
+                        const uint64_t x = o8 >> 16;
+                        const uint32_t e = (uint32_t)__builtin_ctzll(~x | (1ull << 48)) >> 3;  // 6: none
+                        ext = e == 6u;
+                        if (!ext && p + e >= end) {
                             code = HH_ERR_UNEXPECTED_EOF;
                             pos = ilen;
                             return;
                         }
-                        mlen += 255u * e + (uint32_t)((x >> (8 * e)) & 0xffu);
-                        p += e + 1;
-                    } else {
-                        uint64_t m64 = mlen + 255ull * 6;
-                        p += 6;
-                        const int r = p >= end ? 1 : d.ext_slow(p, end, m64, bout != 0);
-                        if (r == 1) {
-                            code = HH_ERR_UNEXPECTED_EOF;
-                            pos = ilen;
-                            return;
+                        mlen += 255u * e + (ext ? 0u : (uint32_t)((x >> (8 * e)) & 0xffu));
+                        p += ext ? 6u : e + 1u;
+                    }
+                } else {
+                    mlen = acc;
+                }
+                if (ext) {
+                    const int r = d.ext_slow(p, end, mlen);
+                    if (r == 1) {
+                        code = HH_ERR_UNEXPECTED_EOF;
+                        pos = ilen;
+                        return;
+                    }
+                    if (r == 2) {
+                        if (bout == 0) {
+                            ip = p;
+                            acc = mlen;
+                            ms = kMatchExt;
                         }
-                        if (r == 2) {  // parse the offset again after the batch
-                            restage = true;
-                            break;
-                        }
-                        if (m64 > 0xffffffffull) {  // more than any capacity
-                            code = HH_ERR_BUFFER_TOO_SMALL;
-                            req = (uint64_t)op + m64;
-                            return;
-                        }
-                        mlen = (uint32_t)m64;
+                        restage = true;
+                        break;
+                    }
+                    if (mlen > 0xffffffffull) {  // more than any capacity
+                        code = HH_ERR_BUFFER_TOO_SMALL;
+                        req = (uint64_t)op + mlen;
+                        return;
                     }
                 }
                 if (mlen > cap - op) {
@@ -1221,8 +1242,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                     return;
                 }
                 ip = p;
-                m_rem = mlen;
-                m_off = off;
+                m_rem = (uint32_t)mlen;
                 ms = kMatch;
             }
             // ms == kMatch: a match whose offset fits the ring reads it

@@ -111,6 +111,27 @@ def test_long_runs_between_short_sequences(decoder, seed):
     check_against_oracle([s for s, _ in items], [c for _, c in items], out_align=seed * 5, out_pad=3)
 
 
+def test_length_extensions_across_stages(decoder):
+    # lengths whose extension bytes end before, at and past one and two input
+    # stages (4 KiB, or 2 KiB with the 8 KiB ring), from several positions in
+    # a stage, whole, cut short, and with too small a capacity
+    stage = 2048 if decoder == "seq8" else 4096
+    rng = np.random.default_rng(stage)
+    streams, caps = [], []
+    for n in (stage - 8, stage + 1, 2 * stage + 9):
+        for at in (0, 1, 100, stage - 70):
+            head = bytes(rng.integers(0, 256, at + 1, dtype=np.uint8))
+            lit = bytes(rng.integers(0, 256, 4096, dtype=np.uint8)) * (n * 255 // 4096 + 1)
+            lit = lit[:15 + 255 * n + at % 255]
+            for s, c in ((_seq(head, 1, 9) + _seq(lit, 60000, 30) + _seq(b"tail5"), at + len(lit) + 45),
+                         (_seq(head, at // 2 + 1, 19 + 255 * n + at) + _seq(b"tail5"), at + 25 + 255 * n + at),
+                         (_seq(head, 1, 9) + _seq(b"", at // 2 + 1, 19 + 255 * n) + _seq(b"tail5"),
+                          at + 34 + 255 * n)):
+                streams += [s, s[:at + 10 + n // 2], s]
+                caps += [c, c, c - 7]
+    check_against_oracle(streams, caps, in_pad=3, out_pad=3)
+
+
 @pytest.mark.parametrize("rho", [0.05, 0.10, 0.15, 0.20])
 def test_sparse_tiles_on_both_routes(rho):
     import haagenti_amd as H
