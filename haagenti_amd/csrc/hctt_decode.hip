@@ -686,16 +686,16 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd(DT, NP)) void hctt_decode_k
 //
 // The input stage holds 8 KiB of a block's compressed bytes (a 16 KiB block
 // is staged in two or three batches of loads): it fits a wave's tile area,
-// which leaves the rest of the LDS to three block buffers (five with the batched decoder, launch_hctt_lz4_fused).
+// which leaves the rest of the LDS to three block buffers (up to five with
+// the batched decoder, see launch_hctt_lz4_fused).
 constexpr uint32_t kFusedStageData = 8 * 1024;
 using FusedRing = ring::RingDec<16384, kFusedStageData, true>;
-using FusedSeq = seq::SeqDec<16384, kFusedStageData - 1024, true>;
+using FusedSeq = seq::SeqDec<16384, kFusedStageData, true>;
 constexpr uint32_t kFusedMax = 16384 - 32;
 constexpr uint32_t kFusedBuf = 16384;  // a block buffer: the decoder's ring
-// a decoder's input stage (the sequence-batched decoder's a KiB shorter, its
-// run table and sequence list after it)
+// a decoder's input stage (the sequence-batched decoder's run table after it)
 constexpr uint32_t kFusedStageRing = FusedRing::kSFront + kFusedStageData + FusedRing::kSPad;
-constexpr uint32_t kFusedStageSeq = FusedSeq::kStageLds + FusedSeq::kTabLds + FusedSeq::kListLds;
+constexpr uint32_t kFusedStageSeq = FusedSeq::kStageLds + FusedSeq::kTabLds;
 constexpr uint32_t kFusedStage = kFusedStageRing > kFusedStageSeq ? kFusedStageRing : kFusedStageSeq;
 static_assert(FusedRing::kSFront == FusedSeq::kSFront, "both decoders' stages start at the same offset");
 constexpr int kFusedMaxWaves = 12;     // 3 per SIMD: 168 registers, tile_body's budget
@@ -948,7 +948,6 @@ __global__ __launch_bounds__(64 * kFusedMaxWaves) void hctt_lz4_fused_kernel(Til
             d.ring = (seq::lds8 *)(size_t)(Fk.buf_off + x * kFusedBuf);
             d.stage = (seq::lds8 *)(size_t)(wbase + FusedSeq::kSFront);
             d.tab = (seq::lds32 *)(size_t)(wbase + FusedSeq::kStageLds);
-            d.list = (seq::lds16 *)(size_t)(wbase + FusedSeq::kStageLds + FusedSeq::kTabLds);
         } else {
             d.ring = rbuf;
             d.stage = stage;

@@ -32,8 +32,7 @@ __global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B) {
     seq::lds8 *lds = (seq::lds8 *)smem;
     d.ring = lds;
     d.tab = reinterpret_cast<seq::lds32 *>(lds + R);
-    d.list = reinterpret_cast<seq::lds16 *>(lds + R + D::kTabLds);
-    d.stage = lds + R + D::kTabLds + D::kListLds + D::kSFront;
+    d.stage = lds + R + D::kTabLds + D::kSFront;
     d.gbuf = B.in;
     d.gsz = B.in_total;
     d.ioff = ioff;

@@ -24,9 +24,9 @@
 //
 // LDS per wave:
 //  * an output ring of R bytes holding the block's latest output.  A match
-//    reads its source from the ring when the source was written at most R
-//    bytes before the end of the current batch (nothing of the batch has
-//    overwritten it), else from the output in global memory, which every
+//    reads its source from the ring when the source was written at most
+//    R - 32 bytes before the end of the current batch (nothing of the batch
+//    has overwritten it), else from the output in global memory, which every
 //    complete 16-byte chunk has reached by then (batches produce at most
 //    R - 64 bytes and complete chunks are written out after each batch);
 //  * an input stage of S bytes of the compressed stream, refilled with
@@ -60,7 +60,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // global read into one flat load, which is not ordered after earlier ds_*
 // writes of other lanes)
 typedef __attribute__((address_space(3))) uint8_t lds8;
-typedef __attribute__((address_space(3))) uint16_t lds16;
 typedef __attribute__((address_space(3))) uint32_t lds32;
 typedef __attribute__((address_space(3))) u32x4 ldsx4;
 
@@ -143,21 +142,22 @@ struct SeqDec {
     static constexpr uint32_t kSFront = 16;                // stage under-read (first chunk of a literal)
     static constexpr uint32_t kSPad = 32;                  // stage over-read (headers, realign)
     static constexpr uint32_t kStageLds = kSFront + S + kSPad;
+    // (with a stage of 8 KiB the table fills a wave's area of the fused
+    // kernel, 12 of which leave room for 3 block buffers)
     static constexpr uint32_t kTabWords = 112;
     static constexpr uint32_t kTabLds = 4 * kTabWords;
     static constexpr uint32_t kList = 256;
-    static constexpr uint32_t kListLds = 2 * kList;
     // batches whose matches may run in any order (match_short): their output
     // bytes each have a bit in the table, and one word after them
     static constexpr uint32_t kShortBytes = 32 * (kTabWords - 1);
     static constexpr uint32_t kShortLit = 32;    // longest literal run copied by one lane
     static constexpr uint32_t kShortMatch = 18;  // longest match without a length extension
-    // ring, table, list, stage (the caller may place them elsewhere)
-    static constexpr uint32_t kLds = R + kTabLds + kListLds + kStageLds;
+    // ring, table, stage (the caller may place them elsewhere)
+    static constexpr uint32_t kLds = R + kTabLds + kStageLds;
 
     lds8 *ring;
     lds32 *tab;           // kTabWords words
-    lds16 *list;          // kList token positions
+    uint32_t list;        // up to kList distances from a token to the next: entry i in byte i / 64 of lane i % 64
     lds8 *stage;          // kSFront bytes of slack before it, kSPad after
     const uint8_t *gbuf;  // whole input buffer: every read is clamped to it
     uint64_t gsz;
@@ -489,17 +489,17 @@ struct SeqDec {
     }
     // Finds the tokens of a run of such sequences from stage offset x0 on,
     // each next token at or before stage offset xe and no window past x_max:
-    // their stage offsets go to the list, their number is returned, x0
-    // becomes the position after the last.
+    // their distances go to the list, their number is returned.
     //
     // The chain of headers is serial; what each link costs is kept small.
     // 256 stage bytes at a time, register r of lane l holds where the next
     // token is if one starts at byte 64 r + l (a multiple of 64 first), so a
     // sequence is one readlane by the position itself and a bit set in a
-    // scalar mask; the positions then go to the list 64 at a time.
-    __device__ __forceinline__ uint32_t walk(uint32_t &x0, uint32_t xe, uint32_t x_max) const {
+    // scalar mask; the distances then go to the list 64 at a time.
+    __device__ __forceinline__ uint32_t walk(uint32_t x, uint32_t xe, uint32_t x_max) {
         constexpr uint32_t kStop = 0xffffu;  // no short sequence here
-        uint32_t n = 0, x = x0;
+        uint32_t n = 0;
+        list = 0;
         bool on = true;
         while (on && n + 96u <= kList && x <= x_max) {
             const uint32_t wb = x & ~63u;
@@ -509,7 +509,7 @@ struct SeqDec {
                 const uint32_t p = wb + 64u * r + (uint32_t)lane;
                 const uint32_t a = p < xe ? p : 0u;
                 const uint32_t k = short_dist(stage[a], stage[a + 1u]);
-                nx[r] = k != 0u && p + k <= xe ? p + k : kStop;
+                nx[r] = k - 1u < 255u && p + k <= xe ? p + k : kStop;
             }
             uint64_t mask[4];
             uint32_t o = x, last = x;
@@ -539,14 +539,18 @@ struct SeqDec {
             x = o;
 #pragma unroll
             for (uint32_t r = 0; r < 4; r++) {
-                const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask[r] >> 32),
-                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)mask[r], 0u));
-                if ((mask[r] >> lane) & 1ull) list[at] = (uint16_t)(wb + 64u * r + (uint32_t)lane);
-                n += (uint32_t)__builtin_popcountll(mask[r]);
+                // the entries go to lanes n, n + 1, ... (mod 64), a zero from
+                // every other lane to the lanes left
+                const uint32_t c = (uint32_t)__builtin_popcountll(mask[r]);
+                const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask[r] >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mask[r], 0u));
+                const bool in = (mask[r] >> lane) & 1ull;
+                const uint32_t at = n + (in ? below : c + (uint32_t)lane - below);
+                const uint32_t k = nx[r] - (wb + 64u * r + (uint32_t)lane);
+                list |= (uint32_t)__builtin_amdgcn_ds_permute((int)(4u * at), in ? (int)(k << (8u * (at >> 6))) : 0);
+                n += c;
             }
         }
-        wave_sync();
-        x0 = x;
         return n;
     }
 
@@ -593,7 +597,7 @@ struct SeqDec {
         const uint64_t own = live ? ((1ull << n) - 1ull) << (r & 31u) : 0ull;
         const uint32_t ow = r >> 5;
         tab[lane] = 0u;
-        if (lane < (int)(kTabWords - 64u)) tab[64 + lane] = 0u;
+        if (kTabWords > 64u && lane < (int)(kTabWords - 64u)) tab[64 + lane] = 0u;
         wave_sync();
         if (live) __hip_atomic_fetch_or(&tab[ow], (uint32_t)own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (own >> 32)
@@ -750,8 +754,13 @@ struct SeqDec {
         // that: the ring serves sources from rlo on, 32 bytes after its
         // start, and what lies before is in the written-out output.
         const int32_t rlo = (int32_t)(op + a0) - (int32_t)R + 32;
-        if (op - op_b >= 256u * nsl) {
-            // runs of 128 bytes or more on average: one run per pass
+        // Long runs one per pass: 128 bytes each on average or, where every
+        // match is short (and shares a pass with others), literals of about
+        // 640.  Sparse tiles' blocks hold such: at 256 for both a fused layer
+        // of hidden size 512 and retention 0.21 took 73 us, now 63; half-zeroed
+        // data with long matches 49 us (600 blocks of 16 KiB) at 640, 44 at 256.
+        const bool tiny_m = ballot(ml > kShortMatch) == 0;
+        if (op - op_b >= (tiny_m ? 640u : 256u) * nsl) {
             for (uint32_t i = 0; i < nsl; i++) {
                 const uint32_t v = rdl(vl, i), n = rdl(ll, i);
                 if (n > 0) lit_serial(v, n, rdl(ls, i));
@@ -769,7 +778,7 @@ struct SeqDec {
             return;
         }
         // short runs: all literal runs of the batch at once, then the matches
-        const bool short_m = op - op_b <= kShortBytes && ballot(ml > kShortMatch) == 0;
+        const bool short_m = tiny_m && op - op_b <= kShortBytes;
         FarSrc fs;
         if (short_m && !LDS) {
             // far sources are final: their loads run beside the literal copies
@@ -880,8 +889,9 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
     uint64_t acc = 0;  // kLitExt, kMatchExt: the length so far
     d.hv = 0;
     d.hb = 0;
-    // the list of short sequences: next entry, entries, stage offset after them
-    uint32_t li = 0, ln = 0, lx = 0;
+    d.list = 0;
+    // the list of short sequences: next entry (the one at ip), entries
+    uint32_t li = 0, ln = 0;
     d.pf_on = false;
     if (end == 0) return;
     if (!staged)
@@ -928,16 +938,19 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                             if (D::walkable((uint32_t)d.peek8(fp), we - (fp - d.sb))) {
                                 // (their output is at least their input: no
                                 // token past the batch's budget)
-                                lx = fp - d.sb;
-                                ln = d.walk(lx, we, lx + (fl - fo));
+                                ln = d.walk(fp - d.sb, we, fp - d.sb + (fl - fo));
                                 li = 0;
                             }
                         }
                         if (li < ln) {
                             const uint32_t n = ln - li < 64u - nsl ? ln - li : 64u - nsl;
                             const bool me = lane >= w0 && lane < w0 + n;
+                            const uint32_t e = li + lane - w0;
+                            const uint32_t kw = bperm(d.list, e) >> (8u * ((e >> 6) & 3u));
+                            const uint32_t k = me ? kw & 0xffu : 0u;
+                            const uint32_t ke = scan_add(k);
                             if (me) {
-                                tp = d.list[li + (lane - w0)];
+                                tp = fp - d.sb + ke - k;
                                 const uint32_t token = d.stage[tp], next = d.stage[tp + 1u];
                                 const bool x1 = token >= 0xf0u;
                                 ls = tp + (x1 ? 2u : 1u);
@@ -951,7 +964,7 @@ __device__ __forceinline__ void decode_block(SeqDec<R, S, LDS> &d, uint32_t ilen
                             lt = n;
                             li += n;
                             nsl += n;
-                            fp = d.sb + (li < ln ? rfl((uint32_t)d.list[li]) : lx);
+                            fp += rdl(ke, 63);
                         }
                     }
                     // then the others, one at a time, until a short one

@@ -132,6 +132,17 @@ def test_length_extensions_across_stages(decoder):
     check_against_oracle(streams, caps, in_pad=3, out_pad=3)
 
 
+@pytest.mark.parametrize("mls", [[4, 5, 18], [4, 19], [200, 640]])
+@pytest.mark.parametrize("mean", [128, 250, 330, 640, 660, 1300])
+def test_long_literals(mean, mls):
+    # literals around the averages from which runs are copied one per pass,
+    # with matches that are all short, partly or none
+    rng = np.random.default_rng(mean + len(mls))
+    items = [stream(rng, 60 + i, list(range(mean - 100, mean + 100)), mls, [1, 3, 17, 800, 3000, 4090, 8000])
+             for i in range(16)]
+    check_against_oracle([s for s, _ in items], [c for _, c in items], out_align=7, out_pad=3)
+
+
 @pytest.mark.parametrize("rho", [0.05, 0.10, 0.15, 0.20])
 def test_sparse_tiles_on_both_routes(rho):
     import haagenti_amd as H
