@@ -699,7 +699,6 @@ constexpr uint32_t kFusedStageSeq = FusedSeq::kStageLds + FusedSeq::kTabLds;
 constexpr uint32_t kFusedStage = kFusedStageRing > kFusedStageSeq ? kFusedStageRing : kFusedStageSeq;
 static_assert(FusedRing::kSFront == FusedSeq::kSFront, "both decoders' stages start at the same offset");
 constexpr int kFusedMaxWaves = 12;     // 3 per SIMD: 168 registers, tile_body's budget
-constexpr int kFusedSeqWaves = 8;      // with the batched decoder (launch_hctt_lz4_fused)
 constexpr uint32_t kFusedMaxBufs = 5;
 constexpr uint32_t kFusedLdsMax = 160u * 1024u;
 constexpr uint32_t kSpinLimit = 1u << 24;  // polls of about 64 cycles each
@@ -743,7 +742,7 @@ constexpr uint32_t kFusedWaveOff = kFusedFlagsOff + ((4 * kFusedFlagWords + 15u)
 // waves with a whole-tile park each and three block buffers
 static_assert(kFusedWaveOff + 12u * 64u * kParkPitch<HH_BF16> + 3u * kFusedBuf <= kFusedLdsMax,
               "twelve waves and three block buffers fit the LDS");
-static_assert(kFusedWaveOff + kFusedSeqWaves * 64u * kParkPitch<HH_BF16> + 5u * kFusedBuf <= kFusedLdsMax,
+static_assert(kFusedWaveOff + 8u * 64u * kParkPitch<HH_BF16> + 5u * kFusedBuf <= kFusedLdsMax,
               "eight waves and five block buffers fit the LDS");
 
 typedef uint32_t __attribute__((address_space(3))) lds_word;
@@ -1277,7 +1276,7 @@ hipError_t launch_hctt_lz4_fused(const hh_hctt_tensor *tensors, uint32_t n, cons
         F.in_len = d_in_len;
         F.status = d_status;
         F.blk_base = blk;
-        uint32_t max_k = 0, total = 0, nb = 0;
+        uint32_t max_k = 0, min_k = 4096, total = 0, nb = 0, sparse = 0;
         for (; i < n && B.n < (uint32_t)kMaxTensors; i++) {
             const hh_hctt_tensor &T = tensors[i];
             const uint32_t nt = (T.rows / 64) * (T.cols / 64);
@@ -1296,6 +1295,8 @@ hipError_t launch_hctt_lz4_fused(const hh_hctt_tensor *tensors, uint32_t n, cons
             total += nt;
             nb += (nt + tpb[i] - 1) / tpb[i];
             max_k = T.k > max_k ? T.k : max_k;
+            min_k = T.k < min_k ? T.k : min_k;
+            sparse += T.k < 1024u ? nt : 0u;
         }
         if (B.n == 0) continue;
         B.start[B.n] = total;
@@ -1309,18 +1310,32 @@ hipError_t launch_hctt_lz4_fused(const hh_hctt_tensor *tensors, uint32_t n, cons
         const uint32_t obytes = 64 * (dtype == HH_F32 ? kParkPitch<HH_F32> : kParkPitch<HH_BF16>);
         B.vo_bytes = ((vbytes > obytes ? vbytes : obytes) + 15u) & ~15u;
         B.wave_lds = B.vo_bytes > kFusedStage ? B.vo_bytes : (kFusedStage + 15u) & ~15u;
-        // One workgroup per CU: kFusedMaxWaves waves (fewer when their areas
-        // leave room for fewer than 3 block buffers).  With the batched
-        // decoder a block is a long chain on one wave, and what bounds the
-        // launch is how many are decoded at once: 8 waves, which leave room
-        // for 5 buffers (f32 parks: 5 waves and 4).  A Llama-3-8B layer to
-        // bf16, 12 waves and 3 buffers / 10 and 4 / 8 and 5 / 6 and 6:
-        // retention 0.10 754 / 626 / 454 / 491 us, 0.20 418 / 335 / 299 /
-        // 326, 0.10-0.50 402 / 384 / 367 / 386; to f32 at 0.10, 6 and 3 / 5
-        // and 4 / 4 and 5: 718 / 602 / 622.  The ring decoder's short chains
-        // keep 12 (retention 0.30: 173 us, 9 and 4 179, 8 and 5 184).
-        uint32_t nw = seq_decoder ? kFusedSeqWaves : kFusedMaxWaves, nbuf = 0;
-        const uint32_t want = seq_decoder && dtype == HH_F32 ? 4u : 3u;
+        // One workgroup per CU: kFusedMaxWaves waves and 3 block buffers
+        // (fewer waves when their areas leave room for fewer buffers).  The
+        // batched decoder's blocks are long chains on one wave each, and
+        // where those are many what bounds the launch is how many are decoded
+        // at once: 8 waves leave room for 5 buffers, 10 for 4.  A Llama-3-8B
+        // layer to bf16, 12 waves and 3 buffers / 10 and 4 / 8 and 5 / 6 and
+        // 6: retention 0.24 229 / 201 / 195 / 232 us, 0.20 364 / 306 / 280 /
+        // 312, 0.10 713 / 580 / 437 / 492; but where most tiles are dense
+        // their decode wants the waves: q, k, v and o at 0.20, the rest at
+        // 0.60 268 / 282 / 293 / 344, all at 0.30 191 / - / 204 (8 and 5).  So
+        // more buffers from a quarter of sparse tiles on (down at 0.20, the
+        // rest at 0.60: 297 / 252 / 264), as many as a workgroup has blocks
+        // (hidden size 2048, 4 blocks: 0.20 110 / 109 / 118), and 5 for the
+        // longest chains (hidden size 2048, 0.10: 209 / 205 / 190).  To f32,
+        // whose parked tiles are twice as large, 6 and 3 / 5 and 4 / 4 and 5:
+        // 0.24 266 / 274 / 313, 0.20 377 / 364 / 409, 0.10 681 / 570 / 597,
+        // gate and up at 0.20 and the rest at 0.60 347 / 327 / 377, q, k, v
+        // and o 340 / 362 / 398: 4 from half of the tiles on.  The ring
+        // decoder's short chains keep 12 (retention 0.30: 173 us, 9 and 4
+        // 179, 8 and 5 184).
+        const uint32_t cus = (uint32_t)(num_cus > 0 ? num_cus : 256), per_wg = (nb + cus - 1) / cus;
+        uint32_t nw = kFusedMaxWaves, nbuf = 0, want = 3;
+        if (seq_decoder && dtype == HH_F32)
+            want = per_wg >= 4 && 2ull * sparse >= total ? 4 : 3;
+        else if (seq_decoder && 4ull * sparse >= total)
+            want = per_wg >= 5 || min_k < 512 ? 5 : per_wg == 4 ? 4 : 3;
         for (;;) {
             const uint32_t used = kFusedWaveOff + nw * B.wave_lds;
             nbuf = used < kFusedLdsMax ? (kFusedLdsMax - used) / kFusedBuf : 0u;
@@ -1336,7 +1351,7 @@ hipError_t launch_hctt_lz4_fused(const hh_hctt_tensor *tensors, uint32_t n, cons
         const uint32_t threads = 64u * nw;
         // workgroup g takes blocks g, g + grid, ...: at most kFusedMaxRange
         // of them (the bitmaps' size)
-        uint32_t grid = (uint32_t)(num_cus > 0 ? num_cus : 256);
+        uint32_t grid = cus;
         if (grid > nb) grid = nb;
         if ((nb + grid - 1) / grid > kFusedMaxRange) grid = (nb + kFusedMaxRange - 1) / kFusedMaxRange;
         const u32x4 *basis = reinterpret_cast<const u32x4 *>(d_basis);
