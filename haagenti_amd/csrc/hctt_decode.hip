@@ -1319,23 +1319,23 @@ hipError_t launch_hctt_lz4_fused(const hh_hctt_tensor *tensors, uint32_t n, cons
         // 6: retention 0.24 229 / 201 / 195 / 232 us, 0.20 364 / 306 / 280 /
         // 312, 0.10 713 / 580 / 437 / 492; but where most tiles are dense
         // their decode wants the waves: q, k, v and o at 0.20, the rest at
-        // 0.60 268 / 282 / 293 / 344, all at 0.30 191 / - / 204 (8 and 5).  So
-        // more buffers from a quarter of sparse tiles on (down at 0.20, the
-        // rest at 0.60: 297 / 252 / 264), as many as a workgroup has blocks
-        // (hidden size 2048, 4 blocks: 0.20 110 / 109 / 118), and 5 for the
-        // longest chains (hidden size 2048, 0.10: 209 / 205 / 190).  To f32,
-        // whose parked tiles are twice as large, 6 and 3 / 5 and 4 / 4 and 5:
-        // 0.24 266 / 274 / 313, 0.20 377 / 364 / 409, 0.10 681 / 570 / 597,
-        // gate and up at 0.20 and the rest at 0.60 347 / 327 / 377, q, k, v
-        // and o 340 / 362 / 398: 4 from half of the tiles on.  The ring
-        // decoder's short chains keep 12 (retention 0.30: 173 us, 9 and 4
-        // 179, 8 and 5 184).
+        // 0.60 268 / 282 / 293 / 344, all at 0.30 191 / - / 204.  So 8 and 5
+        // from a quarter of sparse tiles on (down at 0.20, the rest at 0.60:
+        // 297 / 252 / 264) where a workgroup has 5 blocks (hidden size 2048,
+        // 4 blocks: 0.20 110 / 109 / 118), and for the longest chains (hidden
+        // size 2048, 0.10: 209 / 205 / 190; k at 0.10, the rest at 0.30: 313
+        // / 310 / 291).  To f32, whose parked tiles are twice as large, 6 and
+        // 3 / 5 and 4 / 4 and 5: 0.24 266 / 274 / 313, 0.20 377 / 364 / 409,
+        // 0.10 681 / 570 / 597, gate and up at 0.20 and the rest at 0.60 347
+        // / 327 / 377, q, k, v and o 340 / 362 / 398: 4 from half of the tiles
+        // on, below retention 0.215.  The ring decoder's short chains keep 12
+        // (retention 0.30: 173 us, 9 and 4 179, 8 and 5 184).
         const uint32_t cus = (uint32_t)(num_cus > 0 ? num_cus : 256), per_wg = (nb + cus - 1) / cus;
         uint32_t nw = kFusedMaxWaves, nbuf = 0, want = 3;
         if (seq_decoder && dtype == HH_F32)
-            want = per_wg >= 4 && 2ull * sparse >= total ? 4 : 3;
-        else if (seq_decoder && 4ull * sparse >= total)
-            want = per_wg >= 5 || min_k < 512 ? 5 : per_wg == 4 ? 4 : 3;
+            want = min_k < 880 && per_wg >= 4 && 2ull * sparse >= total ? 4 : 3;
+        else if (seq_decoder)
+            want = min_k < 512 || (per_wg >= 5 && 4ull * sparse >= total) ? 5 : 3;
         for (;;) {
             const uint32_t used = kFusedWaveOff + nw * B.wave_lds;
             nbuf = used < kFusedLdsMax ? (kFusedLdsMax - used) / kFusedBuf : 0u;
