@@ -369,6 +369,15 @@ namespace {
 // against 195 us, at 2048 (8,448) 210 against 223, at 4096 (37,888) 244
 // against 326.
 constexpr uint64_t kSplitTiles = 6144;
+// Retention (k) of the sparsest tensor below which a layer is split: chains
+// shorter than those end with the dense blocks anyway, in a large layer the
+// sooner for the waves that share a CU.  One stream / split, k at 0.24, 0.23,
+// 0.22, 0.21 and 0.20, the rest at 0.30: hidden size 2048 (11,520 dense tiles)
+// 83 / 95, 88 / 95, 96 / 91, 107 / 92, 117 / 101 us to bf16, 104 / 109, 106 /
+// 109, 116 / 109, 126 / 109, 136 / 108 to f32; hidden size 4096 (52,224) 199 /
+// 219, 200 / 225, 210 / 226, 213 / 225, 227 / 224 and 286 / 306, 285 / 294,
+// 290 / 293, 293 / 293, 312 / 292.
+constexpr uint32_t split_k(uint64_t dense_tiles) { return dense_tiles < 24576 ? 920 : 880; }
 
 // Whether a call on `s` may use the context's stream beside it: not while
 // either is being captured, so that the context's stream never belongs to a
@@ -415,7 +424,7 @@ struct SparseSplit {
 
     // Whether the call takes this route: the decoder not chosen by the
     // caller, valid tensors of both kinds, enough dense tiles to hide a
-    // chain behind, and nothing the halves write (tile bytes, weights,
+    // chain behind and chains long enough to be worth it, and nothing the halves write (tile bytes, weights,
     // statuses) shared with what the other one reads or writes.
     bool plan(const hh_context *ctx, const uint8_t *d_in, size_t in_total, const uint64_t *d_in_off,
               const uint32_t *d_in_len, const uint8_t *d_scratch, const uint64_t *d_out_off,
@@ -434,6 +443,7 @@ struct SparseSplit {
                                    span(d_status, sizeof(hh_block_status) * (uint64_t)nblocks)};
         std::vector<Span> dtiles, stiles, douts, souts;
         uint64_t ndense = 0, nsparse = 0;
+        uint32_t min_k = 4096;
         for (uint32_t i = 0; i < n; i++) {
             size_t nt = 0;
             if (hh::check_hctt_tensor(tensors[i], &nt) != HH_OK) return false;
@@ -441,11 +451,12 @@ struct SparseSplit {
             const bool sp = tensors[i].k < 1024u;
             (sp ? sparse : dense).push_back(tensors[i]);
             (sp ? nsparse : ndense) += nt;
+            min_k = tensors[i].k < min_k ? tensors[i].k : min_k;
             (sp ? stiles : dtiles).push_back(span(tensors[i].d_tiles, nt * (uint64_t)hh_hctt_tile_bytes(tensors[i].k)));
             (sp ? souts : douts).push_back(span(tensors[i].d_out, 4096ull * nt * esz));
             if (tensors[i].d_tile_status) (sp ? souts : douts).push_back(span(tensors[i].d_tile_status, 4ull * nt));
         }
-        if (nsparse == 0 || ndense < kSplitTiles || ndense + nsparse > 0xffffffffu) return false;
+        if (ndense < kSplitTiles || min_k >= split_k(ndense) || ndense + nsparse > 0xffffffffu) return false;
         fixed.insert(fixed.end(), stiles.begin(), stiles.end());
         for (const Span &t : dtiles)
             for (const Span &f : fixed)
