@@ -71,6 +71,9 @@ struct hh_context {
     // lock keeps one thread's event records and waits together.
     std::mutex side_lock;
     hipEvent_t fork = nullptr, join = nullptr;
+    hipStream_t side_of = nullptr;      // the stream whose half went to `stream` last
+    bool last_split = false;            // there was a call that may be split,
+    hipStream_t last_stream = nullptr;  // the latest on this stream
 };
 
 namespace hh {

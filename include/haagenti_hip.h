@@ -252,9 +252,11 @@ int32_t hh_hctt_decode_batch(hh_context *ctx, const hh_hctt_tensor *tensors, uin
  * status record per block in d_status), then the tensors, whose d_tiles point
  * into d_scratch, are decoded (hh_hctt_decode_batch semantics); all of it is
  * ordered on `stream` with no host synchronization (a large layer with
- * tensors on both sides of k = 1024 decodes the two kinds beside each other,
- * one of them on hh_context_stream(), after the work queued on `stream`, which
- * waits for it; not while either stream is captured).
+ * tensors on both sides of k = 1024, the sparsest well below, decodes the two
+ * kinds beside each other, one of them on hh_context_stream(), after the work
+ * queued on `stream`, which waits for it; not while either stream is captured,
+ * where hh_context_stream() is busy with other work, or where the context's
+ * last such call was on another stream).
  * This is what
  * HctReader::decompress_all (haagenti-hct/src/tensor.rs:417-515) followed by
  * GpuDecompressor::decompress_batch_to_gpu (haagenti-cuda/src/decompress.rs:

@@ -189,3 +189,61 @@ def test_streams_threads_and_capture():
         assert same(calls[0].results(), want[0])
         calls[2].run()
         assert same(calls[2].results(), want[2])
+
+
+def test_calls_on_other_streams_do_not_wait():
+    # neither for what a caller has put on the context's stream, nor for an
+    # earlier call on a stream that is still busy
+    T = G.torch()
+    ctx = G.ctx()
+    calls = [Call(layer([DENSE, SPARSE, SPARSE2], 5 + i), ctx=ctx) for i in range(2)]
+    want = [general(c) for c in calls]
+    m = T.randn(8192, 8192, device="cuda")
+
+    def busy(stream):
+        # about 100 ms: long after the layer's call has returned and run
+        with T.cuda.stream(stream):
+            for _ in range(12):
+                m @ m
+            return stream.record_event()
+
+    def beside(*others):
+        # a stream that shares no hardware queue with those
+        for _ in range(16):
+            x, free = T.cuda.Stream(), True
+            for o in others:
+                done = busy(o)
+                with T.cuda.stream(x):
+                    T.zeros(1, device="cuda")
+                x.synchronize()
+                free = free and not done.query()
+                T.cuda.synchronize()
+            if free:
+                return x
+        pytest.skip("every stream shares a hardware queue with one of those")
+
+    own = T.cuda.ExternalStream(ctx.stream)
+    s = beside(own)
+    calls[0].clear()
+    T.cuda.synchronize()
+    for _ in range(8):          # each after the halves of the one before
+        calls[0].run(s.cuda_stream)
+    assert same(calls[0].results(), want[0])
+    calls[0].clear()
+    T.cuda.synchronize()
+    done = busy(own)
+    calls[0].run(s.cuda_stream)
+    s.synchronize()
+    assert not done.query()
+    assert same(calls[0].results(), want[0])
+    t = beside(s, own)
+    for c in calls:
+        c.clear()
+    T.cuda.synchronize()
+    done = busy(s)
+    calls[0].run(s.cuda_stream)
+    calls[1].run(t.cuda_stream)
+    t.synchronize()
+    assert not done.query()
+    for c, w in zip(calls, want):
+        assert same(c.results(), w)
