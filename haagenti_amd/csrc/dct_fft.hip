@@ -741,8 +741,6 @@ int32_t tables_for(hh_context *ctx, const Plan &P, hipStream_t s, const float2 *
         t.tab = nullptr;
         return from_hip(e);
     }
-    t.n = P.N;
-    t.stamp = ++ctx->dct_stamp;
     TabPlan TP;
     TP.L = P.L;
     TP.N = P.N;
@@ -752,6 +750,8 @@ int32_t tables_for(hh_context *ctx, const Plan &P, hipStream_t s, const float2 *
                        reinterpret_cast<float2 *>(t.tab), TP);
     e = hipGetLastError();
     if (e != hipSuccess) return from_hip(e);
+    t.n = P.N;  // found from here on
+    t.stamp = ++ctx->dct_stamp;
     *out = reinterpret_cast<const float2 *>(t.tab);
     return HH_OK;
 }

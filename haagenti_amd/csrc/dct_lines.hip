@@ -1046,8 +1046,6 @@ int32_t tables_for(hh_context *ctx, const LinePlan &P, hipStream_t s, const floa
         v->tab = nullptr;
         return from_hip(e);
     }
-    v->n = P.N;
-    v->stamp = ++ctx->dct_stamp;
     LineTabArgs TP;
     TP.N = P.N;
     TP.nr = P.nr;
@@ -1057,6 +1055,8 @@ int32_t tables_for(hh_context *ctx, const LinePlan &P, hipStream_t s, const floa
                        reinterpret_cast<float2 *>(v->tab), TP);
     e = hipGetLastError();
     if (e != hipSuccess) return from_hip(e);
+    v->n = P.N;  // found from here on
+    v->stamp = ++ctx->dct_stamp;
     *out = reinterpret_cast<const float2 *>(v->tab);
     return HH_OK;
 }

@@ -440,12 +440,12 @@ static int32_t planes_for(hh_context *ctx, uint32_t n, int kind, hipStream_t s, 
         b.hl = nullptr;
         return from_hip(e);
     }
-    b.n = n;
-    b.kind = kind;
-    b.stamp = ++ctx->dct_stamp;
     e = kind == 2 ? launch_dct_basis_split_planes(b.hl, b.hl + plane, n, s)
                   : launch_dct_basis_planes(b.hl, b.hl + plane, n, kind == 1, s);
     if (e != hipSuccess) return from_hip(e);
+    b.n = n;  // found from here on
+    b.kind = kind;
+    b.stamp = ++ctx->dct_stamp;
     *hi = b.hl;
     *lo = b.hl + plane;
     return HH_OK;

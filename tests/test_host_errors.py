@@ -1,0 +1,60 @@
+"""Error paths of the entry points on a stand-in HIP runtime (host_hip.cpp,
+no GPU): an allocation or a kernel launch fails, and the call reports it,
+waits for the copies it has queued from memory that goes away with it, and
+leaves nothing half made for the next call."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, sys
+hip = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
+hip.host_hip_calls.restype = C.c_char_p
+sys.path[:0] = [{root!r}, {here!r}]
+import numpy as np
+import haagenti_amd as H
+ctx = H.HipContext(0)
+def calls():
+    return hip.host_hip_calls().decode().split("\\n")[:-1]
+def launches(name):
+    return [c for c in calls() if name in c]
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "libhost_hip.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-o", so, os.path.join(HERE, "host_hip.cpp")], check=True)
+
+    def run(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE.format(so=so, root=os.path.dirname(HERE), here=HERE) + code],
+                           capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stderr[-3000:]
+    return run
+
+
+@pytest.mark.parametrize("rows,cols,route,kernel", [
+    (8, 12, "auto", "lines_tables_kernel"),
+    (64, 17920, "auto", "fft_tables_kernel"),
+    (64, 24, "dense", "basis"),
+])
+def test_tables_of_a_failed_launch_are_not_kept(host, rows, cols, route, kernel):
+    host(f"""
+x = np.zeros(2 * {rows * cols} + 4, np.float32)
+at = (x.ctypes.data + 15) & ~15
+to = at + 4 * {rows * cols}
+for n in (1, 2):                        # the tables of the first and of the second side fail
+    ctx = H.HipContext(0)
+    ctx.set_dct_route({route!r})
+    hip.host_hip_fail({kernel!r}.encode(), n)
+    rc = H._lib.hh_dct_2d(ctx.handle, at, {rows}, {cols}, to, None)
+    assert rc != H.OK and launches({kernel!r})[n - 1:] == launches("failed"), calls()
+    hip.host_hip_fail(b"", 0)
+    rc = H._lib.hh_dct_2d(ctx.handle, at, {rows}, {cols}, to, None)
+    assert rc == H.OK and len(launches({kernel!r})) == 3 - n, calls()
+""")
