@@ -147,6 +147,13 @@ bool unwrap_zstd(const uint8_t *&data, size_t &len, hh::HostBytes &hold) {
     return true;
 }
 
+// The end of a call that waits for its work, also after an error: what it has
+// queued may still read the caller's bytes, its own or the staging buffer.
+int32_t finish(int32_t rc, hipStream_t s) {
+    const hipError_t e = hipStreamSynchronize(s);
+    return rc != HH_OK ? rc : from_hip(e);
+}
+
 // IDCT of d_dense into d_out (dtype), with d_tmp as the GEMM intermediate;
 // d_dense is overwritten for 16-bit outputs; f16_exact when its values came
 // from f16 coefficients.
@@ -397,8 +404,7 @@ int32_t spectral_decode(hh_context *ctx, const Spectral &S, bool pinned, bool up
             const hh::Hct3Frag F{d_bits, d_bits + align16((size_t)S.bm), S.ntot};
             rc = hh::hct3_decode_lines(ctx, &F, 1, S.f32c != 0, S.h, S.w, out_dtype, d_out, s);
         }
-        const hipError_t e = hipStreamSynchronize(s);  // also after an error: the staging buffer is free again
-        if (rc == HH_OK) rc = from_hip(e);
+        rc = finish(rc, s);
         if (rc == HH_OK && status) status->written = S.n;
         return rc;
     }
@@ -413,8 +419,7 @@ int32_t spectral_decode(hh_context *ctx, const Spectral &S, bool pinned, bool up
     float *d_tmp = reinterpret_cast<float *>(base + mat);
     rc = scatter_layers(layers, S.n, S.f32c, d_dense, base + 2 * mat, s);
     if (rc == HH_OK) rc = inverse_to(ctx, d_dense, d_tmp, S.h, S.w, out_dtype, d_out, s, !S.f32c);
-    const hipError_t e = hipStreamSynchronize(s);
-    if (rc == HH_OK) rc = from_hip(e);
+    rc = finish(rc, s);
     if (rc == HH_OK && status) status->written = S.n;
     return rc;
 }
@@ -438,9 +443,7 @@ int32_t hh_hct3_coefficients(hh_context *ctx, const uint8_t *data, size_t len, u
     rc = ensure_scratch(ctx, stage_bytes(total, mc, 0));
     if (rc != HH_OK) return rc;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    rc = scatter_layers(layers, total, 0, d_coeffs, reinterpret_cast<uint8_t *>(ctx->d_scratch), s);
-    if (rc != HH_OK) return rc;
-    return from_hip(hipStreamSynchronize(s));
+    return finish(scatter_layers(layers, total, 0, d_coeffs, reinterpret_cast<uint8_t *>(ctx->d_scratch), s), s);
 }
 
 int32_t hh_hct3_decompress(hh_context *ctx, const uint8_t *data, size_t len, const uint64_t *shape,
@@ -468,9 +471,7 @@ int32_t hh_hct3_decompress(hh_context *ctx, const uint8_t *data, size_t len, con
         uint8_t *d_data = reinterpret_cast<uint8_t *>(ctx->d_scratch);
         hipError_t e = hipMemcpyAsync(d_data, data, len, hipMemcpyHostToDevice, s);
         if (e != hipSuccess) return from_hip(e);
-        rc = decode_lines(ctx, layers, data, d_data, rows, cols, out_dtype, d_out, s);
-        if (rc != HH_OK) return rc;
-        return from_hip(hipStreamSynchronize(s));
+        return finish(decode_lines(ctx, layers, data, d_data, rows, cols, out_dtype, d_out, s), s);
     }
     if (eo_candidate(layers, rows, cols, out_dtype, d_out)) {
         // the same on the even / odd split or the long-row FFT
@@ -481,9 +482,7 @@ int32_t hh_hct3_decompress(hh_context *ctx, const uint8_t *data, size_t len, con
         uint8_t *d_data = base + st;
         hipError_t e = hipMemcpyAsync(d_data, data, len, hipMemcpyHostToDevice, s);
         if (e != hipSuccess) return from_hip(e);
-        rc = decode_eo(ctx, layers, data, d_data, rows, cols, out_dtype, d_out, base, s);
-        if (rc != HH_OK) return rc;
-        return from_hip(hipStreamSynchronize(s));
+        return finish(decode_eo(ctx, layers, data, d_data, rows, cols, out_dtype, d_out, base, s), s);
     }
     const size_t mat = align16((size_t)total * sizeof(float));
     rc = ensure_scratch(ctx, 2 * mat + stage_bytes(total, mc, 0));
@@ -493,8 +492,7 @@ int32_t hh_hct3_decompress(hh_context *ctx, const uint8_t *data, size_t len, con
     float *d_tmp = reinterpret_cast<float *>(base + mat);
     rc = scatter_layers(layers, total, 0, d_dense, base + 2 * mat, s);
     if (rc == HH_OK) rc = inverse_to(ctx, d_dense, d_tmp, rows, cols, out_dtype, d_out, s, true);
-    if (rc != HH_OK) return rc;
-    return from_hip(hipStreamSynchronize(s));
+    return finish(rc, s);
 }
 
 int32_t hh_hct3_decompress_device(hh_context *ctx, const uint8_t *h_data, const uint8_t *d_data, size_t len,

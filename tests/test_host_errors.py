@@ -58,3 +58,29 @@ for n in (1, 2):                        # the tables of the first and of the sec
     rc = H._lib.hh_dct_2d(ctx.handle, at, {rows}, {cols}, to, None)
     assert rc == H.OK and len(launches({kernel!r})) == 3 - n, calls()
 """)
+
+
+@pytest.mark.parametrize("rows,cols,route,fail", [
+    (64, 48, "auto", "row_counts_kernel"),      # the fragments read by the row pass
+    (64, 48, "auto", "lines_tables_kernel"),
+    (512, 1024, "dense", "amax_f16_kernel"),    # the even / odd split of the bases
+    (64, 24, "dense", "basis"),                 # the dense products
+    (64, 24, "coefficients", "scatter"),        # no transform
+])
+def test_a_failed_decode_waits_for_its_copies(host, rows, cols, route, fail):
+    host(f"""
+from test_oracle_hct3 import container, random_fragment
+data = container([random_fragment(np.random.default_rng(1), {rows * cols}, 0.3)])
+out = np.zeros({rows * cols} + 4, np.float32)
+at = (out.ctypes.data + 15) & ~15
+hip.host_hip_fail({fail!r}.encode(), 1)
+if {route!r} == "coefficients":
+    rc = H._lib.hh_hct3_coefficients(ctx.handle, data, len(data), {rows * cols}, at, None)
+else:
+    ctx.set_dct_route({route!r})
+    arr, rank = H._shape_arr([{rows}, {cols}])
+    rc = H._lib.hh_hct3_decompress(ctx.handle, data, len(data), arr, rank, H.F32, at, None)
+c = calls()
+assert rc != H.OK and launches("failed"), c
+assert "copy" in c and "synchronize" in c[len(c) - c[::-1].index("copy"):], c
+""")
