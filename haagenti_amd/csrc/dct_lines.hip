@@ -50,9 +50,14 @@ constexpr uint32_t kMaxPrime = 127;
 constexpr uint32_t kMaxFrags = 16;
 constexpr uint32_t kQB = 8;             // output pairs per wave task of a prime pass
 constexpr uint32_t kMaxTasks = 2;       // wave tasks of a prime pass held in registers
+constexpr uint32_t kFewButterflies = 64;  // below them a prime pass has a thread per output pair
+constexpr uint32_t kFewPairs = 4;         // of them per thread, at most (63 butterflies, 63 pairs)
 
 enum : int { kSrcRows = 0, kSrcPanels = 1, kSrcFrags = 2 };
 enum : int { kDstPanels = 3 };          // else the dtype of a row-major result
+// prime passes of a kernel: none, of at least kFewButterflies butterflies, any
+// (each its own kernel: the last one's registers cost the others up to 5 %)
+enum : int { kPrimesNone = 0, kPrimesMany = 1, kPrimesAny = 2 };
 
 struct Lines {
     const float *in;
@@ -302,6 +307,10 @@ __device__ __forceinline__ float2 tab_at(const float2 *t, uint32_t so, uint32_t 
 __device__ __forceinline__ uint32_t mod_p(uint32_t x, uint32_t p, float invp) {
     return x - (uint32_t)(((float)x + 0.5f) * invp) * p;
 }
+// x / p for a multiple x of p, as above
+__device__ __forceinline__ uint32_t mod_div(uint32_t x, uint32_t p, float invp) {
+    return (uint32_t)(((float)x + 0.5f) * invp);
+}
 // LDS slot of point x of pair pr
 __device__ __forceinline__ uint32_t slot(const Lines &A, uint32_t x, uint32_t pr) {
     return ((x + (x >> A.psh)) << A.pcs) + pr;
@@ -392,7 +401,11 @@ __device__ __forceinline__ void fft_pass(float2 *buf, const Lines &A, uint32_t p
 // A pass of prime radix r > 7 as direct sums (y_q and y_{r-q} share their
 // products, see dft_odd): a_m and b_m are formed in place, then each wave
 // task sums kQB outputs q for 64 butterflies, the roots of unity scalar.
-template <bool INV>
+// With fewer butterflies most of those lanes would idle through 63 steps one
+// after the other: there every output pair (q, butterfly) has a thread.  127 x
+// 127 85 -> 13 us (the dense products 41), 381^2 107 -> 16 (79), 1016^2 152 ->
+// 35 (163).
+template <bool INV, int PR>
 __device__ __forceinline__ void prime_pass(float2 *buf, const Lines &A, uint32_t r, uint32_t p,
                                            const float2 *__restrict__ ptab, const float2 *__restrict__ rt) {
     uint32_t T = blockDim.x, tid = threadIdx.x, nb = A.N / r;
@@ -400,24 +413,70 @@ __device__ __forceinline__ void prime_pass(float2 *buf, const Lines &A, uint32_t
     const uint32_t lane = tid & 63u, nbt = nb << A.pcs, pm = (1u << A.pcs) - 1u, H = (r - 1u) / 2u;
     const float invp = 1.0f / (float)p;
     const uint32_t rstep = (nb + (nb >> A.psh)) << A.pcs, wstep = (p + (p >> A.psh)) << A.pcs;
-    for (uint32_t m = 1; m <= H; m++) {
-        for (uint32_t g = tid; g < nbt; g += T) {
-            const uint32_t i = g >> A.pcs, s = slot(A, i, g & pm);
-            float2 a = buf[s + m * rstep], b = buf[s + (r - m) * rstep];
-            if (p > 1) {
-                const uint32_t k = mod_p(i, p, invp);
-                float2 ta = tab_at(ptab, (m - 1) * p, k), tb = tab_at(ptab, (r - m - 1) * p, k);
-                if (!INV) {
-                    ta.y = -ta.y;
-                    tb.y = -tb.y;
-                }
-                a = cmul(a, ta);
-                b = cmul(b, tb);
+    // a_m and b_m of butterfly g
+    auto pair_up = [&](uint32_t m, uint32_t g) {
+        const uint32_t i = g >> A.pcs, s = slot(A, i, g & pm);
+        float2 a = buf[s + m * rstep], b = buf[s + (r - m) * rstep];
+        if (p > 1) {
+            const uint32_t k = mod_p(i, p, invp);
+            float2 ta = tab_at(ptab, 0, (m - 1) * p + k), tb = tab_at(ptab, 0, (r - m - 1) * p + k);
+            if (!INV) {
+                ta.y = -ta.y;
+                tb.y = -tb.y;
             }
-            buf[s + m * rstep] = cadd(a, b);
-            buf[s + (r - m) * rstep] = rot90<INV>(csub(a, b));
+            a = cmul(a, ta);
+            b = cmul(b, tb);
         }
+        buf[s + m * rstep] = cadd(a, b);
+        buf[s + (r - m) * rstep] = rot90<INV>(csub(a, b));
+    };
+    if (PR == kPrimesAny && nbt < kFewButterflies) {
+        // a thread per output pair (q, butterfly) instead: the sums over m
+        // are the chain that counts
+        const uint32_t all = H * nbt;
+        const float invn = 1.0f / (float)nbt;
+        for (uint32_t e = tid; e < all; e += T) {
+            const uint32_t g = mod_p(e, nbt, invn);
+            pair_up(mod_div(e - g, nbt, invn) + 1u, g);
+        }
+        __syncthreads();
+        float2 re[kFewPairs], im[kFewPairs], y0[kFewPairs];
+#pragma unroll
+        for (uint32_t t = 0; t < kFewPairs; t++) {
+            const uint32_t e = tid + t * T;
+            if (e >= all) continue;
+            const uint32_t g = mod_p(e, nbt, invn), q = mod_div(e - g, nbt, invn) + 1u;
+            const uint32_t s = slot(A, g >> A.pcs, g & pm);
+            re[t] = y0[t] = buf[s];
+            im[t] = make_float2(0.0f, 0.0f);
+            uint32_t idx = 0;
+#pragma unroll 4
+            for (uint32_t m = 1; m <= H; m++) {
+                const float2 a = buf[s + m * rstep], b = buf[s + (r - m) * rstep];
+                idx += q;
+                idx = idx >= r ? idx - r : idx;
+                const float2 cs = rt[idx];
+                y0[t] = cadd(y0[t], a);
+                re[t] = make_float2(__builtin_fmaf(cs.x, a.x, re[t].x), __builtin_fmaf(cs.x, a.y, re[t].y));
+                im[t] = make_float2(__builtin_fmaf(cs.y, b.x, im[t].x), __builtin_fmaf(cs.y, b.y, im[t].y));
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t t = 0; t < kFewPairs; t++) {
+            const uint32_t e = tid + t * T;
+            if (e >= all) continue;
+            const uint32_t g = mod_p(e, nbt, invn), q = mod_div(e - g, nbt, invn) + 1u;
+            const uint32_t i = g >> A.pcs, k = mod_p(i, p, invp), s = slot(A, (i - k) * r + k, g & pm);
+            if (q == 1) buf[s] = y0[t];
+            buf[s + q * wstep] = cadd(re[t], im[t]);
+            buf[s + (r - q) * wstep] = csub(re[t], im[t]);
+        }
+        __syncthreads();
+        return;
     }
+    for (uint32_t m = 1; m <= H; m++)
+        for (uint32_t g = tid; g < nbt; g += T) pair_up(m, g);
     __syncthreads();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = T >> 6;
     const uint32_t wb = (nbt + 63u) / 64u, nq = (H + kQB - 1u) / kQB;
@@ -511,7 +570,7 @@ __global__ __launch_bounds__(256) void row_counts_kernel(RowCounts P) {
 }
 
 // One pass: the transforms of 2 PC lines per workgroup.
-template <bool INV, int SRC, int DST>
+template <bool INV, int SRC, int DST, int PR>
 __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
     extern __shared__ float2 buf[];
     const uint32_t N = A.N, T = blockDim.x, tid = threadIdx.x;
@@ -815,7 +874,7 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
             case 5: fft_pass<5, INV, false, false>(buf, A, p, pt, load16, store16); break;
             case 7: fft_pass<7, INV, false, false>(buf, A, p, pt, load16, store16); break;
             default:
-                prime_pass<INV>(buf, A, r, p, pt, A.rt + roff);
+                if constexpr (PR != kPrimesNone) prime_pass<INV, PR>(buf, A, r, p, pt, A.rt + roff);
                 roff += r;
                 break;
         }
@@ -954,6 +1013,7 @@ bool make_line_plan(uint32_t N, LinePlan &P) {
 // threads.
 struct Split {
     uint32_t pcs, threads, lds;
+    int primes;
 };
 uint32_t lds_points(uint32_t N, uint32_t psh, uint32_t pcs) { return (N + (psh == 4u ? N / 16u : 0u)) << pcs; }
 
@@ -966,11 +1026,16 @@ bool make_split(const LinePlan &P, uint32_t lines, bool frags, uint32_t want_gro
     // (threads per pair of lines a multiple of 16, see lines_kernel)
     const uint32_t unit = pcs == 3 ? 128u : 64u;
     uint32_t T = ((pts + kPerThread - 1u) / kPerThread + unit - 1u) / unit * unit;
+    S.primes = kPrimesNone;
     for (uint32_t q = 0; q < P.nr; q++) {
         const uint32_t r = P.r[q];
         if (r <= 8 || r == 16) continue;
-        const uint32_t tasks = (((P.N / r) << pcs) + 63u) / 64u * (((r - 1u) / 2u + kQB - 1u) / kQB);
-        const uint32_t need = (tasks + kMaxTasks - 1u) / kMaxTasks * 64u;
+        const uint32_t nbt = (P.N / r) << pcs, H = (r - 1u) / 2u;
+        const uint32_t tasks = (nbt + 63u) / 64u * ((H + kQB - 1u) / kQB);
+        const uint32_t few = nbt * H < 1024u ? nbt * H : 1024u;
+        const int kind = nbt < kFewButterflies ? kPrimesAny : kPrimesMany;
+        S.primes = S.primes < kind ? kind : S.primes;
+        const uint32_t need = nbt < kFewButterflies ? few : (tasks + kMaxTasks - 1u) / kMaxTasks * 64u;
         T = T < need ? (need + unit - 1u) / unit * unit : T;
     }
     if (T > 1024u) return false;
@@ -1079,13 +1144,21 @@ void fill(Lines &A, const LinePlan &P, const Split &S, uint32_t lines, const flo
     A.coef_f32 = 0;
 }
 
-template <bool INV, int SRC, int DST>
-hipError_t launch_lines(const Lines &A, const Split &S, uint32_t grid, hipStream_t s) {
-    hipError_t e = hipFuncSetAttribute((const void *)lines_kernel<INV, SRC, DST>,
+template <bool INV, int SRC, int DST, int PR>
+hipError_t launch_lines_pr(const Lines &A, const Split &S, uint32_t grid, hipStream_t s) {
+    hipError_t e = hipFuncSetAttribute((const void *)lines_kernel<INV, SRC, DST, PR>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)S.lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((lines_kernel<INV, SRC, DST>), dim3(grid), dim3(S.threads), S.lds, s, A);
+    hipLaunchKernelGGL((lines_kernel<INV, SRC, DST, PR>), dim3(grid), dim3(S.threads), S.lds, s, A);
     return hipGetLastError();
+}
+template <bool INV, int SRC, int DST>
+hipError_t launch_lines(const Lines &A, const Split &S, uint32_t grid, hipStream_t s) {
+    switch (S.primes) {
+        case kPrimesNone: return launch_lines_pr<INV, SRC, DST, kPrimesNone>(A, S, grid, s);
+        case kPrimesMany: return launch_lines_pr<INV, SRC, DST, kPrimesMany>(A, S, grid, s);
+        default: return launch_lines_pr<INV, SRC, DST, kPrimesAny>(A, S, grid, s);
+    }
 }
 
 // Whether the columns go to the result by way of panels of their own and

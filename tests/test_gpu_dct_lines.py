@@ -57,6 +57,22 @@ def test_transforms_vs_f64(rows, cols):
             assert bool((out[off + rows * cols:] == 7).all()) and (off == 0 or float(out[0]) == 7)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 31), (127, 1), (11, 13), (127, 127), (8001, 3), (2, 8001), (8128, 3),
+                                       (1651, 140), (140, 2431), (961, 600), (1016, 300), (3, 16002)])
+def test_prime_passes(rows, cols):
+    # one to 63 butterflies to a workgroup (a thread per output pair; 3,969
+    # pairs, four to a thread, at 63 x 127) and 64 (one more: wave tasks), both
+    # in one length (127 x 13, 11 x 13 x 17), and passes after others
+    T, c = G.torch(), G.ctx()
+    x = T.randn(rows, cols, device="cuda", generator=T.Generator(device="cuda").manual_seed(rows + cols))
+    br, bc, xd = basis64(rows), basis64(cols), x.double()
+    out = T.empty(rows * cols, device="cuda")
+    for f, ref in ((c.dct_2d, br @ xd @ bc.t()), (c.idct_2d, br.t() @ xd @ bc)):
+        f(x, rows, cols, out, stream=G.stream())
+        e = float((out.view(rows, cols).double() - ref).norm() / ref.norm())
+        assert e <= REL, e
+
+
 @pytest.mark.parametrize("shape", [(97, 131), (64, 1000), (1000, 77), (1, 3000), (130, 2048)])
 def test_fragments_whose_rows_start_inside_a_byte(shape):
     rng = np.random.default_rng(shape[0])
