@@ -502,22 +502,21 @@ struct SparseSplit {
     }
 
     hipError_t launch(hh_context *ctx, hh::Lz4Batch B, int32_t dtype, hipStream_t s) const {
-        B.nrange = (uint32_t)runs.size();
-        for (uint32_t i = 0; i < B.nrange; i++) {
-            B.lo[i] = runs[i].lo;
-            B.hi[i] = runs[i].hi;
+        hh::Lz4Ranges r;
+        r.n = (uint32_t)runs.size();
+        for (uint32_t i = 0; i < r.n; i++) {
+            r.lo[i] = runs[i].lo;
+            r.hi[i] = runs[i].hi;
         }
         ctx->side_of = s;
         hipError_t e = hipEventRecord(ctx->fork, s);
         if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, ctx->fork, 0);
         if (e != hipSuccess) return e;
         // the chains start first and go straight on to their tiles
-        B.part = hh::kPartIn;
         B.first = first;
-        const hipError_t ea = hh::launch_lz4_batch(B, HH_LZ4_SEQ, s);
-        B.part = hh::kPartOut;
+        const hipError_t ea = hh::launch_lz4_seq_in(B, r, s);
         B.first = 0;
-        e = hh::launch_lz4_batch(B, HH_LZ4_RING4, ctx->stream);
+        e = hh::launch_lz4_ring_out(B, r, ctx->stream);
         if (e == hipSuccess)
             e = hh::launch_hctt_decode(dense.data(), (uint32_t)dense.size(), dtype, ctx->d_basis, ctx->num_cus,
                                        ctx->stream, dtype == HH_F32 ? 1u : 4u);

@@ -183,9 +183,6 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float f) {
 hipError_t launch_dequant_int4(const uint8_t *d_q, size_t n, size_t nscale_groups,
                                int dtype, void *d_out, int num_cus, hipStream_t s);
 
-// which of a batch's blocks a launch decodes (Lz4Batch::part)
-enum : uint32_t { kPartAll = 0, kPartIn = 1, kPartOut = 2 };
-constexpr uint32_t kLz4Ranges = 8;
 // One batched LZ4 decode: block i reads in[in_off[i], +in_len[i]) (ranges
 // outside [0, in_total) are reported as HH_ERR_INVALID_ARGUMENT) and writes
 // at most out_cap[i] bytes at out + out_off[i]; a block whose output range
@@ -208,19 +205,29 @@ struct Lz4Batch {
     // the block the sequence-batched launch starts with (the others follow,
     // wrapping around), see lz4_first_block
     uint32_t first = 0;
-    // kPartIn: only the blocks whose output lies inside one of the nrange
-    // address ranges [lo, hi); kPartOut: only the others (ring and
-    // sequence-batched decoders)
-    uint32_t part = kPartAll, nrange = 0;
+};
+// Which of a batch's blocks a launch decodes: all, or only those whose output
+// lies inside (not inside) one of a few address ranges [lo, hi).  Kernels of
+// their own: the ranges and their test cost a launch of one block 0.4 of its
+// 11.7 us.
+constexpr uint32_t kLz4Ranges = 8;
+struct Lz4Ranges {
+    uint32_t n = 0;
     uint64_t lo[kLz4Ranges] = {}, hi[kLz4Ranges] = {};
 };
-__device__ __forceinline__ bool lz4_in_part(const Lz4Batch &B, uint64_t oofs, uint32_t ocap) {
-    if (B.part == kPartAll) return true;
-    const uint64_t a = (uint64_t)(uintptr_t)B.out + oofs;
-    bool in = false;
-    for (uint32_t i = 0; i < B.nrange; i++) in = in || (a >= B.lo[i] && a <= B.hi[i] && ocap <= B.hi[i] - a);
-    return in == (B.part == kPartIn);
-}
+struct Lz4All {
+    __device__ __forceinline__ bool takes(const uint8_t *, uint32_t) const { return true; }
+};
+template <bool IN>
+struct Lz4Some {
+    Lz4Ranges r;
+    __device__ __forceinline__ bool takes(const uint8_t *out, uint32_t cap) const {
+        const uint64_t a = (uint64_t)(uintptr_t)out;
+        bool in = false;
+        for (uint32_t i = 0; i < r.n; i++) in = in || (a >= r.lo[i] && a <= r.hi[i] && cap <= r.hi[i] - a);
+        return in == IN;
+    }
+};
 
 // Batched LZ4 with the decoder `decoder` (hh_lz4_decoder; HH_LZ4_AUTO is
 // resolved by the caller): the sequence-batched decoder (lz4_seq.hip), the
@@ -260,6 +267,10 @@ inline uint32_t lz4_first_block(const hh_hctt_tensor *tensors, uint32_t n, uint3
 }
 hipError_t launch_lz4_seq(const Lz4Batch &B, uint32_t ring_kib, hipStream_t s);
 hipError_t launch_lz4_ring(const Lz4Batch &B, uint32_t ring_kib, hipStream_t s);
+// the two halves of a split layer (4 KiB rings): the blocks inside the ranges
+// with the sequence-batched decoder, the others with the ring decoder
+hipError_t launch_lz4_seq_in(const Lz4Batch &B, const Lz4Ranges &r, hipStream_t s);
+hipError_t launch_lz4_ring_out(const Lz4Batch &B, const Lz4Ranges &r, hipStream_t s);
 
 hipError_t launch_xxh3_batch(const uint8_t *d_data, size_t data_len, const uint64_t *d_off,
                              const uint32_t *d_len, uint32_t n, uint64_t *d_out, hipStream_t s);

@@ -5,8 +5,8 @@
 namespace hh {
 namespace {
 
-template <uint32_t R, uint32_t S>
-__global__ __launch_bounds__(64) void lz4_ring_kernel(Lz4Batch B) {
+template <uint32_t R, uint32_t S, class PART>
+__global__ __launch_bounds__(64) void lz4_ring_kernel(Lz4Batch B, PART part) {
     using D = ring::RingDec<R, S>;
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x;
@@ -20,7 +20,7 @@ __global__ __launch_bounds__(64) void lz4_ring_kernel(Lz4Batch B) {
     const uint32_t ilen = B.in_len[b];
     const uint64_t oofs = B.out_off[b];
     const uint32_t ocap = B.out_cap[b];
-    if (!lz4_in_part(B, oofs, ocap)) return;
+    if (!part.takes(B.out + oofs, ocap)) return;
     const bool out_ok = oofs <= B.out_total && (uint64_t)ocap <= B.out_total - oofs;
     uint8_t *out = B.out + oofs;
     D d;
@@ -64,13 +64,13 @@ __global__ __launch_bounds__(64) void lz4_ring_kernel(Lz4Batch B) {
     }
 }
 
-template <uint32_t R, uint32_t S>
-hipError_t launch_ring(const Lz4Batch &B, hipStream_t s) {
+template <uint32_t R, uint32_t S, class PART = Lz4All>
+hipError_t launch_ring(const Lz4Batch &B, hipStream_t s, const PART &part = PART{}) {
     constexpr uint32_t lds = ring::RingDec<R, S>::kLds;
-    hipError_t e = hipFuncSetAttribute((const void *)lz4_ring_kernel<R, S>,
+    hipError_t e = hipFuncSetAttribute((const void *)lz4_ring_kernel<R, S, PART>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((lz4_ring_kernel<R, S>), dim3(B.nblocks), dim3(64), lds, s, B);
+    hipLaunchKernelGGL((lz4_ring_kernel<R, S, PART>), dim3(B.nblocks), dim3(64), lds, s, B, part);
     return hipGetLastError();
 }
 
@@ -84,6 +84,11 @@ hipError_t launch_lz4_ring(const Lz4Batch &B, uint32_t ring_kib, hipStream_t s) 
         case 32: return launch_ring<32768, 4096>(B, s);
         default: return launch_ring<4096, 4096>(B, s);
     }
+}
+
+hipError_t launch_lz4_ring_out(const Lz4Batch &B, const Lz4Ranges &r, hipStream_t s) {
+    if (B.nblocks == 0) return hipSuccess;
+    return launch_ring<4096, 4096>(B, s, Lz4Some<false>{r});
 }
 
 }  // namespace hh

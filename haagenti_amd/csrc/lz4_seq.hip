@@ -1,12 +1,14 @@
 // Batched raw-LZ4 block decoder: one wavefront per block, sequences parsed
 // in batches and copied lane-parallel (the decoder is in lz4_seq.hpp).
+#include <type_traits>
+
 #include "lz4_seq.hpp"
 
 namespace hh {
 namespace {
 
-template <uint32_t R, uint32_t S>
-__global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B) {
+template <uint32_t R, uint32_t S, class PART>
+__global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B, PART part) {
     using D = seq::SeqDec<R, S, false>;
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x;
@@ -21,11 +23,11 @@ __global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B) {
     const uint32_t ilen = B.in_len[b];
     const uint64_t oofs = B.out_off[b];
     const uint32_t ocap = B.out_cap[b];
-    if (!lz4_in_part(B, oofs, ocap)) return;
+    if (!part.takes(B.out + oofs, ocap)) return;
     // beside other kernels (a split layer) the chain issues before them:
     // 217 against 265 us for a Llama-3-8B layer's tensors of retention 0.10
     // and 0.20 (190 with the device to itself)
-    if (B.part == kPartIn) __builtin_amdgcn_s_setprio(3);
+    if constexpr (std::is_same_v<PART, Lz4Some<true>>) __builtin_amdgcn_s_setprio(3);
     const bool out_ok = oofs <= B.out_total && (uint64_t)ocap <= B.out_total - oofs;
     uint8_t *out = B.out + oofs;
     D d;
@@ -69,13 +71,13 @@ __global__ __launch_bounds__(64) void lz4_seq_kernel(Lz4Batch B) {
     }
 }
 
-template <uint32_t R, uint32_t S>
-hipError_t launch_seq(const Lz4Batch &B, hipStream_t s) {
+template <uint32_t R, uint32_t S, class PART = Lz4All>
+hipError_t launch_seq(const Lz4Batch &B, hipStream_t s, const PART &part = PART{}) {
     constexpr uint32_t lds = seq::SeqDec<R, S, false>::kLds;
-    hipError_t e = hipFuncSetAttribute((const void *)lz4_seq_kernel<R, S>,
+    hipError_t e = hipFuncSetAttribute((const void *)lz4_seq_kernel<R, S, PART>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((lz4_seq_kernel<R, S>), dim3(B.nblocks), dim3(64), lds, s, B);
+    hipLaunchKernelGGL((lz4_seq_kernel<R, S, PART>), dim3(B.nblocks), dim3(64), lds, s, B, part);
     return hipGetLastError();
 }
 
@@ -87,6 +89,11 @@ hipError_t launch_lz4_seq(const Lz4Batch &B, uint32_t ring_kib, hipStream_t s) {
         case 8: return launch_seq<8192, 2048>(B, s);
         default: return launch_seq<4096, 4096>(B, s);
     }
+}
+
+hipError_t launch_lz4_seq_in(const Lz4Batch &B, const Lz4Ranges &r, hipStream_t s) {
+    if (B.nblocks == 0) return hipSuccess;
+    return launch_seq<4096, 4096>(B, s, Lz4Some<true>{r});
 }
 
 }  // namespace hh
