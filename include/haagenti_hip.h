@@ -115,7 +115,8 @@ int32_t hh_context_synchronize(hh_context *ctx);
  * HH_OPT_DCT_ROUTE picks the whole-matrix transform of hh_idct_2d,
  * hh_dct_2d and the HCT3 decode entries (hh_dct_route): HH_DCT_AUTO (the
  * default) takes the FFT route when both sides allow it, the dense MFMA
- * products otherwise.
+ * products otherwise, and so does HH_DCT_FFT; HH_DCT_DENSE the products for
+ * every shape.
  * HH_OPT_PIPELINE_ROUTE picks how hh_pipeline_submit decodes a unit's
  * tensors (hh_pipeline_route): HH_PIPE_AUTO (the default) decodes each
  * tensor with k >= 1024 whose blocks hold whole tiles in the fused launch
@@ -133,7 +134,7 @@ typedef enum hh_pipeline_route { HH_PIPE_AUTO = 0, HH_PIPE_TWO_LAUNCH = 1, HH_PI
 typedef enum hh_dct_route {
     HH_DCT_AUTO = 0,
     HH_DCT_DENSE = 1, /* split-f16 MFMA products against cached bases, O(n^3) */
-    HH_DCT_FFT = 2    /* row transforms through an FFT, O(n^2 log n), where the sides allow it */
+    HH_DCT_FFT = 2    /* transforms of the lines through an FFT, O(n^2 log n), where the sides allow it */
 } hh_dct_route;
 typedef enum hh_lz4_decoder {
     HH_LZ4_AUTO = 0,   /* per entry point, as above */

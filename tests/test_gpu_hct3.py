@@ -11,9 +11,11 @@
   built; 16-bit outputs are the round-to-nearest-even of the f32 result.
 
 Both whole-matrix routes are covered (the context's HH_OPT_DCT_ROUTE): the
-dense split-f16 MFMA products and the FFT route (Makhoul row transforms over
-an f32 FFT in LDS, the route the reference takes above 4096,
-crates/haagenti-cuda/src/dct_gpu.rs:1081,1404-1412)."""
+dense split-f16 MFMA products and the FFT route (the route the reference takes
+above 4096, crates/haagenti-cuda/src/dct_gpu.rs:1081,1404-1412), here with the
+two-pass transforms of sides up to 16384 (csrc/dct_lines.hip, its own edges in
+test_gpu_dct_lines.py) except for one Llama-70B tensor; test_gpu_dct_long.py
+has the longer sides (csrc/dct_fft.hip)."""
 import contextlib
 import struct
 
@@ -165,9 +167,7 @@ def test_decompress_16bit_outputs_and_device_variant():
 @pytest.mark.parametrize("rows,cols", [(64, 64), (1, 77), (77, 1), (37, 53), (200, 120), (512, 512), (1024, 512),
                                        (512, 1536), (192, 2048)])
 def test_idct_dct_2d(rows, cols, way):
-    # against the f64 closed form; "fft" takes the FFT route where both sides
-    # allow it (multiples of 64 whose halves factor into 2, 3, 5, 7) and the
-    # dense route for the others
+    # against the f64 closed form; "fft" takes the two-pass transforms
     T = G.torch()
     rng = np.random.default_rng(rows + 7 * cols)
     c = rng.normal(0, 1, (rows, cols)).astype(np.float32)
@@ -200,15 +200,14 @@ def test_idct_even_odd_split_single_coefficient(rows, cols, k, l):
     assert np.abs(x.cpu().numpy() - ref).max() <= 1e-6
 
 
-# lengths whose halves run radix 8, 4 (64, 192, 1536, 320, 448, 1344), 2
-# (2048: three radix-8 passes and one radix-2 with four butterflies per
-# thread, the widest variant), 3 (192, 1536, 1344), 5 (320, 640), 7 (448,
+# lengths whose passes are of radix 16 (all), 8 (128, 640, 896, 2048), 4 (64,
+# 192, 320, 448, 1344), 2 (1536), 3 (192, 1344, 1536), 5 (320, 640), 7 (448,
 # 896, 1344)
 @pytest.mark.parametrize("rows,cols", [(64, 192), (320, 448), (1536, 640), (896, 1344), (2048, 128)])
 def test_fft_route_single_coefficient_closed_form(rows, cols):
     # C = e_k e_l^T inverts to the outer product of two basis rows, and the
     # forward transform of that product is e_k e_l^T again; k, l include 0,
-    # n/2 and n-1, which the real-to-complex packing pairs specially
+    # n/2 and n-1, which the packing of two lines pairs specially
     T = G.torch()
     with route("fft"):
         for k, l in [(0, 0), (rows // 2, 1), (rows - 1, cols // 2), (7, cols - 1), (rows // 4 + 3, cols // 4)]:
@@ -253,8 +252,8 @@ def test_fft_route_matches_dense_route_4096():
 
 @pytest.mark.parametrize("odd", [False, True])
 def test_fft_route_fragments_scattered_in_the_first_pass(odd):
-    # on the FFT route the first row pass builds each row from the fragments
-    # in LDS: three fragments, the second overwriting part of the first, the
+    # on the FFT route the row pass builds each row from the fragments in LDS:
+    # three fragments, the second overwriting part of the first, the
     # third running out of values; values 2-byte aligned, or read bytewise
     # when the container sits at an odd device address -- against the oracle
     # and the dense route

@@ -1,7 +1,8 @@
 """Error paths of the entry points on a stand-in HIP runtime (host_hip.cpp,
 no GPU): an allocation or a kernel launch fails, and the call reports it,
 waits for the copies it has queued from memory that goes away with it, and
-leaves nothing half made for the next call."""
+leaves nothing half made for the next call.  And which kernels the transforms
+of a shape launch."""
 import os
 import subprocess
 import sys
@@ -83,4 +84,31 @@ else:
 c = calls()
 assert rc != H.OK and launches("failed"), c
 assert "copy" in c and "synchronize" in c[len(c) - c[::-1].index("copy"):], c
+""")
+
+
+def test_routes_of_the_transforms(host):
+    # the two passes up to 16384, rows and transposes above, the dense
+    # products for the lengths neither takes
+    host("""
+from test_gpu_dct_lines import test_transforms_vs_f64 as lines
+from test_gpu_dct_long import FRAGMENTS, SHAPES
+two, rows, dense = "12lines_kernel", "dct_fft_rows_kernel", "dct_gemm"
+shapes = [(s, two) for m in lines.pytestmark if m.name == "parametrize" for s in m.args[1]]
+shapes += [(s, rows) for s in SHAPES + FRAGMENTS] + [((64, 131), dense), ((17000, 64), dense)]
+for (r, c), kernel in shapes:
+    hip.host_hip_fail(b"", 0)
+    assert H._lib.hh_dct_2d(ctx.handle, 16, r, c, 32, None) == H.OK
+    assert H._lib.hh_idct_2d(ctx.handle, 16, r, c, H.F32, 32, None) == H.OK
+    got = {k for k in (two, rows, dense) if launches(k)}
+    assert got == {kernel}, (r, c, calls())
+from test_oracle_hct3 import container, random_fragment
+for (r, c), scatter in zip(FRAGMENTS, (False, False, True, True)):
+    data = container([random_fragment(np.random.default_rng(1), r * c, 0.01)])
+    out = np.zeros(r * c + 4, np.float32)
+    arr, rank = H._shape_arr([r, c])
+    hip.host_hip_fail(b"", 0)
+    assert H._lib.hh_hct3_decompress(ctx.handle, data, len(data), arr, rank, H.F32, (out.ctypes.data + 15) & ~15,
+                                     None) == H.OK
+    assert launches(rows) and bool(launches("hct3_scatter_kernel")) == scatter, (r, c, calls())
 """)
