@@ -716,15 +716,26 @@ def wl_hct3(args, torch, H, O):
         # bytes = the container read once + the bf16 output written once
         alg = len(data) + n * n * 2
         achieved = alg / per / 1e9
+        two_pass = n <= 16384    # longer sides take row transforms and transposes
+        if two_pass:
+            kernel = ("row_counts_kernel + lines_kernel x2 (Makhoul transforms of several rows, then of several "
+                      "columns per workgroup, over an f32 Stockham FFT in LDS; the rows read the fragments and "
+                      "write f32 panels, the columns write bf16)"
+                      + (" + untangle_kernel (panels of columns to rows)" if n > 8192 else ""))
+            # the panels written and read (twice above 8192, where the columns write panels too), the output
+            passes = 4 * n * n * (2 if n <= 8192 else 4) + 2 * n * n
+        else:
+            kernel = ("dct_fft_rows_kernel x2 (Makhoul rows over an f32 Stockham FFT in LDS; the first "
+                      "builds its rows from the fragments in LDS) + transpose_kernel x2 (the second "
+                      "converting to bf16) + bitmap packing, row counts and their scan")
+            # the first row pass's f32 write, the first transpose and the second row pass (read +
+            # write each), the last transpose's f32 read and bf16 write
+            passes = 4 * n * n * 6 + 2 * n * n
         roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": 8000.0, "unit": "GB/s",
-                "frac": round(achieved / 8000.0, 4), "traffic": traffic_for(f"hct3-{n}-fft"),
-                "kernel": ("dct_fft_rows_kernel x2 (Makhoul rows over an f32 Stockham FFT in LDS; the first "
-                           "builds its rows from the fragments in LDS) + transpose_kernel x2 (the second "
-                           "converting to bf16) + bitmap packing, row counts and their scan"),
-                "avg_launch_us": round(per * 1e6, 1), "algorithmic_bytes_per_launch": alg,
-                # the first row pass's f32 write, the first transpose and the second row pass (read +
-                # write each), the last transpose's f32 read and bf16 write
-                "f32_matrix_passes_bytes": 4 * n * n * 6 + 2 * n * n}
+                "frac": round(achieved / 8000.0, 4),
+                "traffic": traffic_for(f"hct3-{n}-two-pass" if two_pass else f"hct3-{n}-fft"),
+                "kernel": kernel, "avg_launch_us": round(per * 1e6, 1), "algorithmic_bytes_per_launch": alg,
+                "f32_matrix_passes_bytes": passes}
         dt = "f32-fft"
     else:
         flop = 4.0 * n ** 3          # the two dense n x n x n products of the transform

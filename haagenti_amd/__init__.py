@@ -901,8 +901,8 @@ class GpuDecompressor:
     """GpuDecompressor (crates/haagenti-cuda/src/decompress.rs:108-443) for HCT
     V3 fragment containers: decompress(), decompress_to_gpu(),
     decompress_batch(), plus reconstruct_coefficients_gpu() (the dense DCT
-    coefficient matrix before the transform).  zstd-framed input raises
-    UNSUPPORTED."""
+    coefficient matrix before the transform).  zstd-framed input is decoded on
+    the host first."""
 
     def __init__(self, ctx=None):
         self.ctx = ctx if ctx is not None else HipContext(0)

@@ -430,7 +430,7 @@ bool may_split(hh_context *ctx, hipStream_t s) {
 // a chain of ~1,400 sequences on one wave (190 us at retention 0.10, three
 // waves to a CU), which one LZ4 launch makes every tile wait for: a
 // Llama-3-8B layer of retention 0.10-0.50 took 326 us that way (LZ4 190,
-// tiles 130), 244 split (chains 217 beside 42 + 146, then 43 for the sparse
+// tiles 130), 235 split (chains 222 beside 48 + 155, then 43 for the sparse
 // tiles).  The dense tiles of 16-bit outputs run in four turns of
 // workgroups: the chains' waves take the place of some of them, which would
 // otherwise start when the others end (238 against 213 us at retention

@@ -929,7 +929,7 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
 
 // The columns' panels (groups of 2 << pcs columns, N points each) to the
 // row-major result: 64 points of 64 columns per workgroup through LDS, rows
-// of 256 or 128 bytes out.  Bound by memory: 14336 x 4096 f32 81 us, 5.8 TB/s
+// of 256 or 128 bytes out.  Bound by memory: 14336 x 4096 f32 85 us, 5.5 TB/s
 // (the device copy reaches 6.3).
 constexpr uint32_t kTileSide = 64, kTileStride = kTileSide + 2;  // even: pairs of columns stay aligned
 template <bool INV, int DST>
@@ -1163,8 +1163,8 @@ hipError_t launch_lines(const Lines &A, const Split &S, uint32_t grid, hipStream
 
 // Whether the columns go to the result by way of panels of their own and
 // untangle_kernel.  A workgroup of two columns (more than 8192 rows) writes 8
-// or 4 bytes of a row: 14336 x 4096 forward 394 us for that pass, against 241
-// to panels and 81 for the tiles; inverse, whole, 489 -> 450 (bf16 437 -> 424).
+// or 4 bytes of a row: 14336 x 4096 forward 394 us for that pass, against 184
+// to panels (241 before panel_share) and 85 for the tiles; inverse, whole, 489 -> 450 (bf16 437 -> 424).
 // Four columns gain nothing (8192 x 4096 232 -> 265), nor do lengths with a
 // prime pass, whose workgroups don't write all at once (11008 x 4096 bf16 498
 // -> 523).

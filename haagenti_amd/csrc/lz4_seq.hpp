@@ -9,12 +9,13 @@
 // What bounds it: one block is one wave's chain of dependent instructions
 // (7-10 cycles each when the wave is alone on its SIMD).  Tiles of 10 %
 // retention make ~1,400 sequences of ~10 bytes a 16 KiB block; a tensor of
-// 652 such blocks took 612 us when every sequence's header was read on its
+// 652 such blocks took 607 us when every sequence's header was read on its
 // own and matches were copied in runs up to the first that reads one of
-// them, 187 us with the tokens found by a walk (about 110 cycles a sequence),
+// them, 174 us with the tokens found by a walk (about 110 cycles a sequence),
 // one lane copying a sequence's literals and its match, and matches going as
-// soon as their own source bytes are there: 3.4 rounds a batch of 64.  At
-// 15 % 259 -> 123 us, at 20 % 95 -> 82 us.
+// soon as their own source bytes are there: 3.5 rounds a batch of 64.  At
+// 15 % 268 -> 128 us, at 20 % 102 -> 88 us, at 24 % (16 long sequences a
+// block) 59 -> 53.
 //
 // Semantics: crates/haagenti-lz4/src/block.rs:261-366 (decompress_block):
 // the same checks in the same order, the same reported positions, the early
