@@ -1180,28 +1180,42 @@ bool through_panels(const LinePlan &Ph) { return Ph.N > kMaxPoints / 2u && Ph.ro
 // pieces of 2 PC columns x G rows; below a line of memory (128 bytes) two
 // share: 4096 x 14336 bf16 375 -> 353 us, 8192^2 459 -> 437 (four: 378, 479).
 // Before untangle_kernel 256 bytes pay, four at most: 14336 x 4096 485 -> 458
-// (two) -> 445 us, 12288 x 3072 334 -> 301 -> 293; eight no more.
-uint32_t panel_share(const LinePlan &Pw, const LinePlan &Ph, const Split &Sw, const Split &Sh) {
+// (two) -> 445 us, 12288 x 3072 334 -> 301 -> 293; eight no more.  Not for
+// f32 results whose rows are a multiple of 32 KiB apart: pieces of 64 bytes
+// are faster beside the columns' stores, 8192^2 546 -> 518 us (518 on rows and
+// transposes, which took it before), 7168 x 8192 434 -> 418, 4608 x 8192 320
+// -> 291, 4096 x 16384 443 -> 424 (others lose: 8064^2
+// 525 -> 546, 7168^2 354 -> 379; with a prime pass, 7936 x 8192, 541 -> 559;
+// pieces of 32 bytes, 5120 x 16384, 616 -> 642).
+uint32_t panel_share(bool inverse, int32_t dtype, const LinePlan &Pw, const LinePlan &Ph, const Split &Sw,
+                     const Split &Sh) {
     const bool through = through_panels(Ph);
     const uint32_t piece = 4u + Sw.pcs + Sh.pcs, want = through ? 8u : 7u, most = through ? 2u : 1u;
+    if (inverse && dtype == HH_F32 && piece == 6u && Pw.N % 8192u == 0 && Ph.roots == 0) return 0u;
     return piece >= want ? 0u : want - piece < most ? want - piece : most;
 }
 
 // The f32 panels of the rows (whole panels) and those of the columns.
-size_t row_panels(const LinePlan &Pw, const LinePlan &Ph, const Split &Sw, const Split &Sh) {
-    const uint32_t g = 2u << (Sw.pcs + panel_share(Pw, Ph, Sw, Sh));
-    return (size_t)((Ph.N + g - 1u) / g * g) * Pw.N;
-}
-size_t panel_elems(const LinePlan &Pw, const LinePlan &Ph, const Split &Sw, const Split &Sh) {
-    const uint32_t g = 2u << Sh.pcs;
-    return row_panels(Pw, Ph, Sw, Sh) + (through_panels(Ph) ? (size_t)((Pw.N + g - 1u) / g * g) * Ph.N : 0u);
+struct Panels {
+    uint32_t msh;      // panel_share
+    size_t rows, all;  // floats
+};
+Panels panels_for(bool inverse, int32_t dtype, const LinePlan &Pw, const LinePlan &Ph, const Split &Sw,
+                  const Split &Sh) {
+    Panels P;
+    P.msh = panel_share(inverse, dtype, Pw, Ph, Sw, Sh);
+    const uint32_t g = 2u << (Sw.pcs + P.msh), gc = 2u << Sh.pcs;
+    P.rows = (size_t)((Ph.N + g - 1u) / g * g) * Pw.N;
+    P.all = P.rows + (through_panels(Ph) ? (size_t)((Pw.N + gc - 1u) / gc * gc) * Ph.N : 0u);
+    return P;
 }
 
 // Both passes of an h x w transform: rows (from d_in, or the fragments in F)
 // to panels in d_mid, columns to d_out, where they don't lie a line of memory
 // side by side by way of panels and tiles.
 int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines *F, float *d_mid, const LinePlan &Pw,
-                   const LinePlan &Ph, const Split &Sw, const Split &Sh, int32_t dtype, void *d_out, hipStream_t s) {
+                   const LinePlan &Ph, const Split &Sw, const Split &Sh, const Panels &M, int32_t dtype, void *d_out,
+                   hipStream_t s) {
     const float2 *tw, *th;
     int32_t rc = tables_for(ctx, Pw, s, &tw);
     if (rc == HH_OK) rc = tables_for(ctx, Ph, s, &th);
@@ -1216,7 +1230,7 @@ int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines
     A.in = d_in;
     A.out = d_mid;
     uint32_t ga = (h + (2u << Sw.pcs) - 1u) >> (Sw.pcs + 1u);
-    A.msh = panel_share(Pw, Ph, Sw, Sh);
+    A.msh = M.msh;
     if (A.msh) {
         A.per_xcd = (((ga + 7u) / 8u - 1u) | ((1u << A.msh) - 1u)) + 1u;
         ga = 8u * A.per_xcd;
@@ -1244,7 +1258,7 @@ int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines
             e = launch_lines<true, kSrcPanels, HH_F32>(B, Sh, grid, s);
         return from_hip(e);
     }
-    float *cols = d_mid + row_panels(Pw, Ph, Sw, Sh);
+    float *cols = d_mid + M.rows;
     B.out = cols;
     e = inverse ? launch_lines<true, kSrcPanels, kDstPanels>(B, Sh, grid, s)
                 : launch_lines<false, kSrcPanels, kDstPanels>(B, Sh, grid, s);
@@ -1302,10 +1316,12 @@ int32_t dct2d_lines(hh_context *ctx, bool inverse, const float *d_in, uint32_t h
     LinePlan Pw, Ph;
     Split Sw, Sh;
     if (!make_plans(ctx, h, w, false, Pw, Ph, Sw, Sh)) return HH_ERR_UNSUPPORTED;
+    const Panels M = panels_for(inverse, out_dtype, Pw, Ph, Sw, Sh);
     uint8_t *mid;
-    int32_t rc = mid_scratch(ctx, panel_elems(Pw, Ph, Sw, Sh) * sizeof(float), s, &mid);
+    int32_t rc = mid_scratch(ctx, M.all * sizeof(float), s, &mid);
     if (rc != HH_OK) return rc;
-    return two_passes(ctx, inverse, d_in, nullptr, reinterpret_cast<float *>(mid), Pw, Ph, Sw, Sh, out_dtype, d_out, s);
+    return two_passes(ctx, inverse, d_in, nullptr, reinterpret_cast<float *>(mid), Pw, Ph, Sw, Sh, M, out_dtype, d_out,
+                      s);
 }
 
 int32_t hct3_decode_lines(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrags, bool coef_f32, uint32_t h,
@@ -1313,7 +1329,8 @@ int32_t hct3_decode_lines(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrag
     LinePlan Pw, Ph;
     Split Sw, Sh;
     if (nfrags == 0 || nfrags > kMaxFrags || !make_plans(ctx, h, w, true, Pw, Ph, Sw, Sh)) return HH_ERR_UNSUPPORTED;
-    const size_t mid_bytes = (panel_elems(Pw, Ph, Sw, Sh) * sizeof(float) + 255u) & ~(size_t)255u;
+    const Panels M = panels_for(true, dtype, Pw, Ph, Sw, Sh);
+    const size_t mid_bytes = (M.all * sizeof(float) + 255u) & ~(size_t)255u;
     uint8_t *mid;
     const uint32_t pitch = (h + 3u) & ~3u;  // each fragment's counts 16-byte aligned
     int32_t rc = mid_scratch(ctx, mid_bytes + (size_t)nfrags * pitch * 4u, s, &mid);
@@ -1336,7 +1353,7 @@ int32_t hct3_decode_lines(hh_context *ctx, const Hct3Frag *frags, uint32_t nfrag
     hipLaunchKernelGGL(row_counts_kernel, dim3((h + 3u) / 4u, nfrags), dim3(256), 0, s, C);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return from_hip(e);
-    return two_passes(ctx, true, nullptr, &F, reinterpret_cast<float *>(mid), Pw, Ph, Sw, Sh, dtype, d_out, s);
+    return two_passes(ctx, true, nullptr, &F, reinterpret_cast<float *>(mid), Pw, Ph, Sw, Sh, M, dtype, d_out, s);
 }
 
 void release_line_tables(hh_context *ctx) {

@@ -57,6 +57,24 @@ def test_transforms_vs_f64(rows, cols):
             assert bool((out[off + rows * cols:] == 7).all()) and (off == 0 or float(out[0]) == 7)
 
 
+@pytest.mark.parametrize("rows,cols", [(2058, 16384), (4116, 8192)])
+def test_rows_32_kib_apart(rows, cols):
+    # f32 results of such rows come from panels of one row workgroup each,
+    # 16-bit ones from panels that two share
+    T, h, c = G.torch(), H(), G.ctx()
+    x = T.randn(rows, cols, device="cuda", generator=T.Generator(device="cuda").manual_seed(rows + cols))
+    inv = T.empty(rows * cols, device="cuda")
+    half = T.empty(rows * cols, dtype=T.bfloat16, device="cuda")
+    for _ in range(2):  # the second with the other's intermediate in place
+        c.idct_2d(x, rows, cols, inv, stream=G.stream())
+        c.idct_2d(x, rows, cols, half, dtype=h.BF16, stream=G.stream())
+        G.sync()
+        assert T.equal(half, inv.to(T.bfloat16))
+    ref = basis64(rows).t() @ x.double() @ basis64(cols)
+    e = float((inv.view(rows, cols).double() - ref).norm() / ref.norm())
+    assert e <= REL, e
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 31), (127, 1), (11, 13), (127, 127), (8001, 3), (2, 8001), (8128, 3),
                                        (1651, 140), (140, 2431), (961, 600), (1016, 300), (3, 16002)])
 def test_prime_passes(rows, cols):
