@@ -70,6 +70,8 @@ struct Lines {
     uint32_t N;       // line length
     uint32_t lines;   // number of lines
     uint32_t gsh;     // log2 of the panels' height G (kSrcPanels)
+    uint32_t ipitch;  // points from a panel to the next (kSrcPanels)
+    uint32_t opitch;  // the same of the output (kDstPanels)
     uint32_t pcs;     // log2 of the pairs of lines per workgroup
     uint32_t psh;     // LDS: point x at slot x + (x >> psh)
     uint32_t per_xcd; // workgroups per XCD (0: not placed)
@@ -611,7 +613,7 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
         if constexpr (SRC == kSrcRows)
             return n;
         else
-            return (((n >> A.gsh) * A.lines) << A.gsh) + (n & (G - 1u));
+            return (((n >> A.gsh) * A.ipitch) << A.gsh) + (n & (G - 1u));
     };
     // input element at scalar offset so + lane offset vo (elements; a matrix
     // has fewer than 2^29)
@@ -628,7 +630,7 @@ __global__ __launch_bounds__(1024) void lines_kernel(Lines A) {
     // the output's steps: elements of a line, and where pair pr's lines are
     const uint32_t osh = A.pcs + A.msh, part = (grp & ((1u << A.msh) - 1u)) << A.pcs;
     const uint32_t ostep = DST == kDstPanels ? 1u << osh : A.lines;
-    const int32_t obase = (int32_t)(DST == kDstPanels ? (((grp >> A.msh) * N) << osh) + part : line0);
+    const int32_t obase = (int32_t)(DST == kDstPanels ? (((grp >> A.msh) * A.opitch) << osh) + part : line0);
     auto opair = [&](uint32_t pr) -> uint32_t { return DST == kDstPanels ? pr : 2u * pr; };
 
     // (k, N - k) pairs, k = 0 with N / 2; a thread's are istep apart (a
@@ -1143,6 +1145,8 @@ void fill(Lines &A, const LinePlan &P, const Split &S, uint32_t lines, const flo
     A.psh = P.psh;
     A.per_xcd = 0;
     A.msh = 0;
+    A.ipitch = lines;
+    A.opitch = P.N;
     A.nr = P.nr;
     A.radix[0] = A.radix[1] = 0;
     for (uint32_t q = 0; q < P.nr; q++) A.radix[q >> 3] |= (uint64_t)P.r[q] << (8u * (q & 7u));
@@ -1198,6 +1202,7 @@ uint32_t panel_share(bool inverse, int32_t dtype, const LinePlan &Pw, const Line
 // The f32 panels of the rows (whole panels) and those of the columns.
 struct Panels {
     uint32_t msh;      // panel_share
+    uint32_t pitch;    // points from a panel of the rows to the next
     size_t rows, all;  // floats
 };
 Panels panels_for(bool inverse, int32_t dtype, const LinePlan &Pw, const LinePlan &Ph, const Split &Sw,
@@ -1205,7 +1210,17 @@ Panels panels_for(bool inverse, int32_t dtype, const LinePlan &Pw, const LinePla
     Panels P;
     P.msh = panel_share(inverse, dtype, Pw, Ph, Sw, Sh);
     const uint32_t g = 2u << (Sw.pcs + P.msh), gc = 2u << Sh.pcs;
-    P.rows = (size_t)((Ph.N + g - 1u) / g * g) * Pw.N;
+    // Large forward transforms leave two points between the panels of the rows:
+    // a column reads one piece of each, of all of which the addresses would
+    // otherwise differ by a multiple of the line length.  8192^2 575 -> 535 us
+    // (552 on rows and transposes, which took it before), 4096 x 16384 492 ->
+    // 437, 4096 x 11008 497 -> 478, 6144 x 4096 157 -> 155 (four, eight and
+    // twelve points: 546, 534, 532; 448, 461, 448; 472, 477, 476; 159, 158,
+    // 158).  Below 2^23 elements the panels stay in the caches (1024 x 4096
+    // 29.5 -> 30.4); inverse transforms read two pieces and lose (4096 x 8192
+    // 196 -> 202 with eight), as do columns in panels of their own (16384^2).
+    P.pitch = Pw.N + (!inverse && !through_panels(Ph) && (uint64_t)Ph.N * Pw.N >= (1u << 23) ? 2u : 0u);
+    P.rows = (size_t)((Ph.N + g - 1u) / g * g) * P.pitch;
     P.all = P.rows + (through_panels(Ph) ? (size_t)((Pw.N + gc - 1u) / gc * gc) * Ph.N : 0u);
     return P;
 }
@@ -1231,6 +1246,7 @@ int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines
     A.out = d_mid;
     uint32_t ga = (h + (2u << Sw.pcs) - 1u) >> (Sw.pcs + 1u);
     A.msh = M.msh;
+    A.opitch = M.pitch;
     if (A.msh) {
         A.per_xcd = (((ga + 7u) / 8u - 1u) | ((1u << A.msh) - 1u)) + 1u;
         ga = 8u * A.per_xcd;
@@ -1244,6 +1260,7 @@ int32_t two_passes(hh_context *ctx, bool inverse, const float *d_in, const Lines
     B.in = d_mid;
     B.out = d_out;
     B.gsh = Sw.pcs + A.msh + 1u;
+    B.ipitch = M.pitch;
     const uint32_t gb = (w + (2u << Sh.pcs) - 1u) >> (Sh.pcs + 1u);
     B.per_xcd = (gb + 7u) / 8u;
     const uint32_t grid = 8u * B.per_xcd;

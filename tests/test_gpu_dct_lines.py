@@ -75,6 +75,20 @@ def test_rows_32_kib_apart(rows, cols):
     assert e <= REL, e
 
 
+@pytest.mark.parametrize("rows,cols", [(2048, 4096), (2047, 4096), (2057, 4095), (1025, 8190), (513, 16384), (8192, 1025),
+                                       (5504, 1533)])
+def test_forward_panels_apart(rows, cols):
+    # from 2^23 elements on (8192 rows at most) there are two points between
+    # the panels of the rows; ragged last panels, prime passes
+    T, c = G.torch(), G.ctx()
+    x = T.randn(rows, cols, device="cuda", generator=T.Generator(device="cuda").manual_seed(rows + cols))
+    out = T.empty(rows * cols, device="cuda")
+    c.dct_2d(x, rows, cols, out, stream=G.stream())
+    ref = basis64(rows) @ x.double() @ basis64(cols).t()
+    e = float((out.view(rows, cols).double() - ref).norm() / ref.norm())
+    assert e <= REL, e
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 31), (127, 1), (11, 13), (127, 127), (8001, 3), (2, 8001), (8128, 3),
                                        (1651, 140), (140, 2431), (961, 600), (1016, 300), (3, 16002)])
 def test_prime_passes(rows, cols):
