@@ -119,3 +119,20 @@ def test_fragments_whose_rows_start_inside_a_byte(shape):
     with route("dense"):
         dense = dec().decompress_to_gpu(data, shape).cpu().numpy()
     assert rel_err(got, dense) <= 2e-5
+
+
+@pytest.mark.parametrize("nfrag", [1, 3, 16])
+@pytest.mark.parametrize("rows,cols", [(3, 16), (64, 64), (1024, 256), (1024, 512), (1027, 300), (300, 700), (2048, 520),
+                                       (1300, 1024), (4100, 64), (9000, 33), (16384, 34)])
+def test_fragments_by_workgroup_size(rows, cols, nfrag):
+    # one to sixteen waves to a workgroup, one to four to a line, with idle
+    # lanes (short lines), ragged last workgroups and several of them to a CU
+    T, c = G.torch(), G.ctx()
+    rng = np.random.default_rng(rows + cols + nfrag)
+    total = rows * cols
+    data = container([random_fragment(rng, total, 0.6 / (f + 2)) for f in range(nfrag)])
+    x = dec().reconstruct_coefficients_gpu(data, total).view(rows, cols).double()
+    ref = basis64(rows).t() @ x @ basis64(cols)
+    got = dec().decompress_to_gpu(data, (rows, cols))
+    e = float((got.view(rows, cols).double() - ref).norm() / ref.norm())
+    assert e <= REL, e
