@@ -1046,21 +1046,24 @@ bool make_split(const LinePlan &P, uint32_t lines, bool frags, uint32_t want_gro
         const uint32_t need = nbt < kFewButterflies ? few : (tasks + kMaxTasks - 1u) / kMaxTasks * 64u;
         T = T < need ? (need + unit - 1u) / unit * unit : T;
     }
-    if (frags) {
-        // Placing a fragment's values is a chain of loads, scans and barriers,
-        // shorter with more waves: a wave a line for the bitmap words, up to
-        // four where every lane still has elements to place, as long as all
-        // workgroups run at once (16 waves to a CU).  1024 x 512 (a wave of
-        // four lines before) 33 -> 22 us, with eight fragments 117 -> 43 (28
-        // and 92 on rows and transposes); 2048^2 43 -> 39, 123 -> 91.  Past
-        // that they wait for each other: 1536^2 with 16 waves 45 us, with 8
-        // 37, 16384 x 64 with 16 62, with 4 42.
-        const uint32_t c = 2u << pcs, groups = (lines + c - 1u) / c;
-        const uint32_t per_cu = (groups + want_groups - 1u) / want_groups, fill = (pts / 2u + 63u) / 64u;
-        uint32_t waves = fill < c ? c : fill < 4u * c ? fill : 4u * c;
-        waves = waves < 16u / per_cu ? waves : 16u / per_cu;
-        T = T < 64u * waves ? 64u * waves / unit * unit : T;
-    }
+    // More waves than the FFT's radix-16 butterflies need, up to one per 64
+    // pairs of points, as long as all workgroups run at once (16 waves to a
+    // CU): a small pass is the latency of its loads and stores.  Four times as
+    // many: 1024 x 512 inverse to f32 18.0 -> 13.5 us (17.7 on rows and
+    // transposes, which took it before), 3072 x 192 20.9 -> 16.1 (20.2), 5120
+    // x 64 19.6 -> 16.7 (18.9); twice: 14.9, 17.3, 17.1.
+    const uint32_t c = 2u << pcs, groups = (lines + c - 1u) / c;
+    const uint32_t per_cu = (groups + want_groups - 1u) / want_groups, fill = (pts / 2u + 63u) / 64u;
+    uint32_t waves = 4u * T / 64u < fill ? 4u * T / 64u : fill;
+    // Placing a fragment's values is a chain of loads, scans and barriers: a
+    // wave a line for the bitmap words, up to four.  1024 x 512 (a wave of
+    // four lines before) 33 -> 22 us, with eight fragments 117 -> 43 (28 and
+    // 92 on rows and transposes); 2048^2 43 -> 39, 123 -> 91.  Past all
+    // running at once they wait for each other: 1536^2 with 16 waves 45 us,
+    // with 8 37, 16384 x 64 with 16 62, with 4 42.
+    if (frags) waves = fill < c ? c : fill < 4u * c ? fill : 4u * c;
+    waves = waves < 16u / per_cu ? waves : 16u / per_cu;
+    T = T < 64u * waves ? 64u * waves / unit * unit : T;
     if (T > 1024u) return false;
     S.pcs = pcs;
     S.threads = T;

@@ -136,3 +136,18 @@ def test_fragments_by_workgroup_size(rows, cols, nfrag):
     got = dec().decompress_to_gpu(data, (rows, cols))
     e = float((got.view(rows, cols).double() - ref).norm() / ref.norm())
     assert e <= REL, e
+
+
+@pytest.mark.parametrize("rows,cols", [(2, 64), (16, 80), (64, 1024), (1024, 192), (512, 1000), (260, 5120), (5120, 64),
+                                       (1030, 514), (4096, 72), (9000, 65), (1376, 513)])
+def test_small_passes_of_many_waves(rows, cols):
+    # more waves than radix-16 butterflies need, with every lane or only some
+    # at work, one to a few workgroups to a CU, a prime pass, panels of columns
+    T, c = G.torch(), G.ctx()
+    x = T.randn(rows, cols, device="cuda", generator=T.Generator(device="cuda").manual_seed(rows + cols))
+    br, bc, xd = basis64(rows), basis64(cols), x.double()
+    out = T.empty(rows * cols, device="cuda")
+    for f, ref in ((c.dct_2d, br @ xd @ bc.t()), (c.idct_2d, br.t() @ xd @ bc)):
+        f(x, rows, cols, out, stream=G.stream())
+        e = float((out.view(rows, cols).double() - ref).norm() / ref.norm())
+        assert e <= REL, e
