@@ -1030,6 +1030,15 @@ bool make_split(const LinePlan &P, uint32_t lines, bool frags, uint32_t want_gro
     while (pcs < 3 && (P.N << (pcs + 1)) <= kMaxPoints) pcs++;
     // fewer lines per workgroup until there is one for every CU
     while (pcs > 0 && (lines + (2u << pcs) - 1u) / (2u << pcs) < want_groups) pcs--;
+    // and where workgroups that have a CU each would leave a last round of up
+    // to three tenths: 5120 x 1536 to bf16 73 -> 64 us (70 on rows and
+    // transposes, which took it before), 5120 x 1280 65 -> 54 (63), 2560^2 60
+    // -> 44; at half a round 1536 x 6144 loses 2 %, and so do single pairs (8192
+    // x 1280 5 %), whose pieces of a row are 8 bytes
+    const uint32_t parts = (lines + (2u << pcs) - 1u) / (2u << pcs);
+    if (pcs > 1 && lds_points(P.N, P.psh, pcs) * 8u > kMaxLds / 2u && parts > want_groups &&
+        10u * parts < 13u * want_groups)
+        pcs--;
     const uint32_t pts = P.N << pcs;
     // (threads per pair of lines a multiple of 16, see lines_kernel)
     const uint32_t unit = pcs == 3 ? 128u : 64u;

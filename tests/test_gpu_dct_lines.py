@@ -151,3 +151,16 @@ def test_small_passes_of_many_waves(rows, cols):
         f(x, rows, cols, out, stream=G.stream())
         e = float((out.view(rows, cols).double() - ref).norm() / ref.norm())
         assert e <= REL, e
+
+
+@pytest.mark.parametrize("rows,cols", [(4096, 1280), (4100, 1280), (5324, 1287), (1280, 4200), (2560, 2562)])
+def test_workgroups_past_one_round(rows, cols):
+    # 256 workgroups and a few more, up to three tenths more
+    T, c = G.torch(), G.ctx()
+    x = T.randn(rows, cols, device="cuda", generator=T.Generator(device="cuda").manual_seed(rows + cols))
+    br, bc, xd = basis64(rows), basis64(cols), x.double()
+    out = T.empty(rows * cols, device="cuda")
+    for f, ref in ((c.dct_2d, br @ xd @ bc.t()), (c.idct_2d, br.t() @ xd @ bc)):
+        f(x, rows, cols, out, stream=G.stream())
+        e = float((out.view(rows, cols).double() - ref).norm() / ref.norm())
+        assert e <= REL, e
