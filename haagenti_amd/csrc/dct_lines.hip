@@ -1064,14 +1064,24 @@ bool make_split(const LinePlan &P, uint32_t lines, bool frags, uint32_t want_gro
     const uint32_t c = 2u << pcs, groups = (lines + c - 1u) / c;
     const uint32_t per_cu = (groups + want_groups - 1u) / want_groups, fill = (pts / 2u + 63u) / 64u;
     uint32_t waves = 4u * T / 64u < fill ? 4u * T / 64u : fill;
-    // Placing a fragment's values is a chain of loads, scans and barriers: a
-    // wave a line for the bitmap words, up to four.  1024 x 512 (a wave of
-    // four lines before) 33 -> 22 us, with eight fragments 117 -> 43 (28 and
-    // 92 on rows and transposes); 2048^2 43 -> 39, 123 -> 91.  Past all
-    // running at once they wait for each other: 1536^2 with 16 waves 45 us,
-    // with 8 37, 16384 x 64 with 16 62, with 4 42.
-    if (frags) waves = fill < c ? c : fill < 4u * c ? fill : 4u * c;
-    waves = waves < 16u / per_cu ? waves : 16u / per_cu;
+    if (frags) {
+        // Placing a fragment's values is a chain of loads, scans and barriers:
+        // a wave a line for the bitmap words, up to four.  1024 x 512 (a wave
+        // of four lines before) 33 -> 22 us, with eight fragments 117 -> 43
+        // (28 and 92 on rows and transposes); 2048^2 43 -> 39, 123 -> 91.
+        // Past all running at once they wait for each other: 1536^2 with 16
+        // waves 42 us, with 8 34, 16384 x 64 with 16 62, with 4 42; but where
+        // the LDS holds one workgroup it gets all 16 (2304^2 with eight
+        // fragments 254 -> 192, rows and transposes 249), and two and a half
+        // to a CU on average have 8 (2560^2 237 -> 183, 205; with 16 196).
+        const uint32_t held = kMaxLds / (lds_points(P.N, P.psh, pcs) * 8u + c * ((P.N + 31u) / 32u) * 8u + 64u);
+        uint32_t at_once = per_cu < held ? per_cu : held > 0 ? held : 1u;
+        at_once = at_once == 3u ? 2u : at_once;
+        waves = fill < c ? c : fill < 4u * c ? fill : 4u * c;
+        waves = waves < 16u / at_once ? waves : 16u / at_once;
+    } else {
+        waves = waves < 16u / per_cu ? waves : 16u / per_cu;
+    }
     T = T < 64u * waves ? 64u * waves / unit * unit : T;
     if (T > 1024u) return false;
     S.pcs = pcs;

@@ -123,7 +123,7 @@ def test_fragments_whose_rows_start_inside_a_byte(shape):
 
 @pytest.mark.parametrize("nfrag", [1, 3, 16])
 @pytest.mark.parametrize("rows,cols", [(3, 16), (64, 64), (1024, 256), (1024, 512), (1027, 300), (300, 700), (2048, 520),
-                                       (1300, 1024), (4100, 64), (9000, 33), (16384, 34)])
+                                       (1300, 1024), (4100, 64), (9000, 33), (16384, 34), (2310, 1152), (600, 5120)])
 def test_fragments_by_workgroup_size(rows, cols, nfrag):
     # one to sixteen waves to a workgroup, one to four to a line, with idle
     # lanes (short lines), ragged last workgroups and several of them to a CU
